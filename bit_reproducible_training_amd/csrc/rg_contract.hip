@@ -20,72 +20,9 @@
 #include "rg_internal.h"
 #include <type_traits>
 #include "repro_gemm_math.h"
+#include "rg_mfma.h"
 
 namespace rg {
-
-// round_to_float for the rare inputs the binary64 paths hand over (|T| near or above 2^53),
-// kept out of line so the epilogue's common path stays short.
-__device__ __noinline__ float round_to_float_rare(int64_t T, int E) {
-    return repro_gemm::round_to_float(T, E);
-}
-
-// T = sum_l lv[l] * 2^(7 (L-1-l)) as an exact int64.
-template <int L>
-__device__ __forceinline__ int64_t combine_levels(const int (&lv)[L]) {
-    int64_t t = 0;
-#pragma unroll
-    for (int l = 0; l < L; ++l) t += (int64_t)lv[l] * ((int64_t)1 << (7 * (L - 1 - l)));
-    return t;
-}
-
-// round_to_float(T, E) for T = combine_levels(lv), with the levels combined in binary64:
-// Horner steps h = 128 h + lv[l] over int32 levels stay below 2^53 in magnitude up to the
-// next-to-last level (|h| < 2^31 (1 + 2^7 + 2^14 + 2^21) < 2^53 for L = 5), so they are
-// exact; the last step is exact when the next-to-last |h| < 2^45 (then |T| < 2^52 + 2^31).
-// Scaling by 2^E is exact in binary64 when f64_scale_exact(E) (every exponent the slicing
-// produces is: |E| <= 2 * 149 + 28), and the conversion to binary32 is the one IEEE rounding
-// (nearest-even, subnormals, -0.0, overflow to infinity). *ok = false when a condition fails;
-// the value is then meaningless and round_to_float(combine_levels(lv), E) is the result.
-template <int L>
-__device__ __forceinline__ float round_levels_try(const int (&lv)[L], int E, bool* ok) {
-    double h = (double)lv[0];
-#pragma unroll
-    for (int l = 1; l + 1 < L; ++l) h = __builtin_fma(h, 128.0, (double)lv[l]);
-    bool exact = repro_gemm::f64_scale_exact(E);
-    if (L > 1) {
-        exact = exact && __builtin_fabs(h) < 0x1p45;
-        h = __builtin_fma(h, 128.0, (double)lv[L - 1]);
-    }
-    *ok = exact;
-    return (float)__builtin_ldexp(h, E);
-}
-
-template <int L>
-__device__ __forceinline__ float round_levels(const int (&lv)[L], int E) {
-    bool ok;
-    const float r = round_levels_try<L>(lv, E, &ok);
-    return __builtin_expect(ok, 1) ? r : round_to_float_rare(combine_levels<L>(lv), E);
-}
-
-// round_to_float(T, E) for an int64 T: repro_gemm::round_to_float_f64 with its rare
-// fallback out of line.
-__device__ __forceinline__ float round_output(int64_t T, int E) {
-    bool ok;
-    const float r = repro_gemm::round_to_float_f64_try(T, E, &ok);
-    return __builtin_expect(ok, 1) ? r : round_to_float_rare(T, E);
-}
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-
-// s_waitcnt on vector-memory operations only: wait until at most n are outstanding.
-#define RG_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
-// s_waitcnt on LDS (and scalar memory) operations only: wait until none is outstanding.
-#define RG_WAIT_LGKMCNT0() __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (0 << 8))
-// Lambdas of the kernels hold references to register arrays: they must be inlined, or the
-// arrays would move to scratch memory.
-#define RG_INLINE __attribute__((always_inline))
-#define RG_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 
 // Wavefronts per SIMD that the block tile's LDS ring allows (blocks per CU x wavefronts per
 // block / 4), capped at 2 unless one block alone needs more (12 wavefronts: 3): the register

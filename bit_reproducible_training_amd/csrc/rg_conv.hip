@@ -14,9 +14,13 @@
 // weights' scale) and keeps the exact int64 T; col2im_round then adds each pixel's terms in
 // int64 (exact, order-free) and rounds once with E = e_image + e_weights - 14 (S - 1).
 //
+// Most forward passes and input gradients take the fused kernels of rg_conv_fused.hip instead, which
+// round the gathered values inside the contraction (fused_plan says which).
+//
 // The packing kernels move fp32 values only (HBM-bound): im2col with zero padding, and the
 // [N][F][OH*OW] <-> [W][F] transposes of dY and Y.
 #include "rg_internal.h"
+#include "rg_conv_fused.h"
 #include "rg_fastdiv.h"
 #include "repro_conv.h"
 #include "repro_gemm_math.h"
@@ -694,6 +698,8 @@ bool direct_preferred(Kind kind, const Geom& g) {
 struct ConvPlan {
     Geom g;
     bool direct;
+    bool fused;      // the fused implicit GEMM (plan f): forward and input gradient
+    FusedPlan f;
     bool implicit;   // forward GEMM reads the im2col matrix through Im2col (no cols buffer)
     Layout L;        // the GEMM (GEMM algorithm only)
     size_t buf0, buf1, gemm, total;
@@ -720,6 +726,18 @@ int conv_plan(Kind kind, const rg_conv_shape* s, int S, int algo, ConvPlan* P) {
         p.total = CONV_ALIGN;  // no scratch; kept non-zero so that every pass takes a buffer
         *P = p;
         return hipSuccess;
+    }
+    if (kind != Kind::GradWeight) {
+        DeviceInfo dev;
+        const int e = query_device(&dev);
+        if (e != hipSuccess) return e;
+        if (!dev.gfx950) return hipErrorNotSupported;
+        if (fused_plan((int)kind, *s, S, dev.num_cus, &p.f)) {
+            p.fused = true;
+            p.total = p.f.total;
+            *P = p;
+            return hipSuccess;
+        }
     }
     rg_config cfg;
     rg_config_init(&cfg);
@@ -841,6 +859,7 @@ int run_pass(Kind kind, const float* a, const float* b, float* out, const rg_con
         return hipGetLastError();
     }
     char* base = static_cast<char*>(workspace);
+    if (p.fused) return fused_launch(p.f, a, b, out, base, stream);
     char* gws = base + p.gemm;
     switch (kind) {
         case Kind::Forward: {
@@ -981,6 +1000,22 @@ int rg_conv2d_algo_ws(int pass, const float* a, const float* b, float* out, cons
     if (!rg::valid_pass(pass)) return hipErrorInvalidValue;
     return rg::run_pass(static_cast<rg::Kind>(pass), a, b, out, g, S, algo, workspace,
                         workspace_bytes, stream);
+}
+
+int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int* info) {
+    if (!g || !info || !rg::valid_pass(pass) || !rg::valid(g, S) || num_cus < 1) return hipErrorInvalidValue;
+    for (int i = 0; i < 8; ++i) info[i] = 0;
+    rg::FusedPlan p;
+    if (pass == RG_CONV_GRAD_WEIGHT || !rg::fused_plan(pass, *g, S, num_cus, &p)) return hipSuccess;
+    info[0] = 1;
+    info[1] = p.patch;
+    info[2] = p.split;
+    info[3] = p.nclass;
+    info[4] = p.cls[0].NS;
+    info[5] = p.cls[0].GW;
+    info[6] = p.cls[0].pxgroups;
+    info[7] = p.tf;
+    return hipSuccess;
 }
 
 }  // extern "C"

@@ -1,0 +1,87 @@
+"""GPU parity of the fused convolution kernels (forward pass and input gradient) with the oracle,
+bit for bit, at the sizes where they can go wrong: blocks and patches that span images and column
+strips, tiles cut by the last position and channel, channel counts off a group of 16, parts along
+k, residue classes of a strided input gradient (some without taps), kernels larger than the image,
+scales past one normal float, NaN and infinities."""
+import numpy as np
+import pytest
+
+from gpu_util import note
+from oracle import oracle as O
+from test_conv_fused_plan import DX, FWD, fused
+from test_gpu_conv import RC, _oracle, _run_algo
+
+pytestmark = pytest.mark.gpu
+
+# shape: (N, C, H, W, F, KH, KW, SY, SX, PY, PX)
+SHAPES = [
+    (2, 16, 8, 8, 16, 3, 3, 1, 1, 1, 1),        # one position past a block
+    (9, 20, 7, 7, 40, 3, 3, 1, 1, 1, 1),        # blocks over several images
+    (1, 16, 20, 112, 40, 3, 3, 1, 1, 1, 1),     # two column strips
+    (1, 18, 9, 131, 16, 3, 3, 1, 1, 0, 1),      # strips with dead columns
+    (1, 40, 30, 30, 24, 5, 5, 1, 1, 2, 2),
+    (2, 33, 12, 12, 16, 2, 2, 1, 1, 0, 0),      # four taps
+    (1, 50, 13, 40, 17, 7, 7, 1, 1, 3, 3),
+    (1, 35, 16, 16, 70, 2, 3, 1, 1, 1, 0),      # six taps, 70 channels (a second tile, ragged)
+    (3, 32, 40, 13, 130, 1, 1, 1, 1, 0, 0),     # one tap
+    (1, 600, 6, 6, 65, 3, 3, 1, 1, 1, 1),       # parts along k
+    (4, 20, 20, 20, 70, 5, 5, 2, 2, 2, 2),      # four residue classes
+    (2, 17, 17, 19, 9, 3, 5, 2, 1, 0, 2),
+    (2, 40, 11, 11, 24, 1, 1, 2, 2, 0, 0),      # classes without taps
+    (1, 16, 3, 3, 16, 3, 3, 1, 1, 3, 3),        # padding wider than the image
+    (2, 16, 3, 4, 20, 9, 9, 1, 1, 4, 4),        # kernel larger than the image
+    (5, 16, 7, 7, 16, 4, 4, 1, 2, 3, 0),
+]
+
+
+def _inputs(shape, seed):
+    N, C, H, W, F, KH, KW = shape[:7]
+    OH, OW = O.conv_out_hw(shape)
+    rng = np.random.default_rng(seed)
+    x = (rng.standard_normal(N * C * H * W) * 2.0 ** rng.integers(-12, 12, N * C * H * W)).astype(np.float32)
+    w = (rng.standard_normal(F * C * KH * KW) * 0.1).astype(np.float32)
+    dy = (rng.standard_normal((N, F * OH * OW)) * 2.0 ** rng.integers(-30, 30, (N, 1))).astype(np.float32)
+    return x, w, dy.ravel()
+
+
+def _check(torch, shape, S, x, w, dy):
+    for kind, a in (("fwd", x), ("dX", dy)):
+        note("fused conv", kind, shape, "S=%d" % S)
+        got = _run_algo(torch, kind, a, w, shape, S, RC.ALGO_GEMM).view(np.uint32).ravel()
+        assert np.array_equal(got, _oracle(kind, a, w, shape, S).view(np.uint32).ravel()), (kind, shape, S)
+
+
+@pytest.mark.parametrize("S", [1, 2, 3])
+def test_fused_matches_oracle(torch_gpu, S):
+    for i, shape in enumerate(SHAPES):
+        _check(torch_gpu, shape, S, *_inputs(shape, 10 * S + i))
+
+
+def test_shapes_cover_the_routes():
+    plans = [(p, fused(p, s)) for s in SHAPES for p in (FWD, DX)]
+    for pass_ in (FWD, DX):
+        mine = [f for p, f in plans if p == pass_ and f["taken"]]
+        assert any(f["patch"] and f["split"] == 1 for f in mine)
+        assert any(f["split"] > 1 for f in mine)
+        assert any(not f["patch"] for f in mine)
+        assert any(f["strips"] > 1 for f in mine)
+        assert {f["tf"] for f in mine} == {1, 2}
+
+
+@pytest.mark.parametrize("what", ["tiny", "huge", "nonfinite"])
+def test_fused_slow_rounding(torch_gpu, what):
+    """Rows whose scale is not one normal float (maxima below 2^-100 or near 2^127) and values
+    that are not finite leave the one-multiply-add rounding."""
+    for shape in (SHAPES[1], SHAPES[9], SHAPES[10]):
+        x, w, dy = _inputs(shape, 77)
+        rng = np.random.default_rng(5)
+        for t in (x, dy):
+            if what == "tiny":
+                t *= np.float32(2.0 ** -125)
+            elif what == "huge":
+                hit = rng.random(t.size) < 0.3
+                t[hit] = np.where(rng.random(hit.sum()) < 0.5, 3e38, -1e38)
+            else:
+                t[rng.integers(0, t.size, 3)] = np.nan
+                t[rng.integers(0, t.size, 2)] = np.inf
+        _check(torch_gpu, shape, 3, x, w, dy)
