@@ -21,7 +21,7 @@ INCLUDE = os.path.join(REPO_DIR, "include")
 BUILD_DIR = os.path.join(CSRC, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "librepro_gemm.so")
 
-SOURCES = ["rg_slice.hip", "rg_contract.hip", "rg_probe.hip", "rg_sum.hip", "rg_conv.hip", "rg_conv_fused.hip",
+SOURCES = ["rg_slice.hip", "rg_contract.hip", "rg_probe.hip", "rg_sum.hip", "rg_conv.hip", "rg_conv_fused.hip", "rg_conv_dw.hip",
            "rg_api.cpp"]
 BINDING_SOURCE = "rg_torch.cpp"
 

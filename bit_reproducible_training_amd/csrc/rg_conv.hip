@@ -20,6 +20,7 @@
 // The packing kernels move fp32 values only (HBM-bound): im2col with zero padding, and the
 // [N][F][OH*OW] <-> [W][F] transposes of dY and Y.
 #include "rg_internal.h"
+#include "rg_conv_dw.h"
 #include "rg_conv_fused.h"
 #include "rg_fastdiv.h"
 #include "repro_conv.h"
@@ -700,6 +701,8 @@ struct ConvPlan {
     bool direct;
     bool fused;      // the fused implicit GEMM (plan f): forward and input gradient
     FusedPlan f;
+    bool dwfused;    // the weight gradient's fused contraction (plan d)
+    DwPlan d;
     bool implicit;   // forward GEMM reads the im2col matrix through Im2col (no cols buffer)
     Layout L;        // the GEMM (GEMM algorithm only)
     size_t buf0, buf1, gemm, total;
@@ -727,12 +730,19 @@ int conv_plan(Kind kind, const rg_conv_shape* s, int S, int algo, ConvPlan* P) {
         *P = p;
         return hipSuccess;
     }
-    if (kind != Kind::GradWeight) {
+    {
         DeviceInfo dev;
         const int e = query_device(&dev);
         if (e != hipSuccess) return e;
         if (!dev.gfx950) return hipErrorNotSupported;
-        if (fused_plan((int)kind, *s, S, dev.num_cus, &p.f)) {
+        if (kind == Kind::GradWeight) {
+            if (dw_plan(*s, S, dev.num_cus, &p.d)) {
+                p.dwfused = true;
+                p.total = p.d.total;
+                *P = p;
+                return hipSuccess;
+            }
+        } else if (fused_plan((int)kind, *s, S, dev.num_cus, &p.f)) {
             p.fused = true;
             p.total = p.f.total;
             *P = p;
@@ -860,6 +870,7 @@ int run_pass(Kind kind, const float* a, const float* b, float* out, const rg_con
     }
     char* base = static_cast<char*>(workspace);
     if (p.fused) return fused_launch(p.f, a, b, out, base, stream);
+    if (p.dwfused) return dw_launch(p.d, a, b, out, base, stream);
     char* gws = base + p.gemm;
     switch (kind) {
         case Kind::Forward: {
@@ -1005,8 +1016,20 @@ int rg_conv2d_algo_ws(int pass, const float* a, const float* b, float* out, cons
 int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int* info) {
     if (!g || !info || !rg::valid_pass(pass) || !rg::valid(g, S) || num_cus < 1) return hipErrorInvalidValue;
     for (int i = 0; i < 8; ++i) info[i] = 0;
+    if (pass == RG_CONV_GRAD_WEIGHT) {
+        rg::DwPlan d;
+        if (!rg::dw_plan(*g, S, num_cus, &d)) return hipSuccess;
+        info[0] = info[1] = 1;
+        info[2] = d.parts;
+        info[3] = d.RC;
+        info[4] = d.NS;
+        info[5] = d.SW;
+        info[6] = d.pxgroups;
+        info[7] = d.tf;
+        return hipSuccess;
+    }
     rg::FusedPlan p;
-    if (pass == RG_CONV_GRAD_WEIGHT || !rg::fused_plan(pass, *g, S, num_cus, &p)) return hipSuccess;
+    if (!rg::fused_plan(pass, *g, S, num_cus, &p)) return hipSuccess;
     info[0] = 1;
     info[1] = p.patch;
     info[2] = p.split;

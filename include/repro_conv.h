@@ -84,7 +84,8 @@ int rg_conv2d_algo_ws(int pass, const float* a, const float* b, float* out, cons
 /* Test hook (no GPU needed): how the MFMA route runs a pass on a device with num_cus compute units.
  * info[0]: 1 when the pass takes a fused kernel, which rounds the gathered values itself (else 0
  * and the rest is 0); info[1]: 1 when that kernel holds source patches in LDS; info[2]: parts along
- * k; info[3]: classes of output positions; info[4], info[5]: column strips and their width;
+ * k; info[3]: classes of output positions (weight gradient: output rows per chunk of its patches);
+ * info[4], info[5]: column strips and their width;
  * info[6]: patch values per channel, in units of 64; info[7]: 32 x 32 tiles per wavefront. 1
  * (invalid value) for a null argument, an unknown pass or an invalid shape. */
 int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int* info);

@@ -26,7 +26,9 @@ def test_routes():
     for pass_ in (FWD, DX):
         p = fused(pass_, resnet)
         assert p["taken"] and p["patch"] and p["split"] == 1, p
-    assert not fused(DW, resnet)["taken"]
+    assert fused(DW, resnet)["taken"]
+    assert not fused(DW, (32, 512, 7, 7, 512, 3, 3, 1, 1, 1, 1))["taken"]    # many filters, few windows
+    assert not fused(DW, (8, 64, 20, 20, 64, 3, 3, 3, 3, 1, 1))["taken"]     # column stride 3
     strided = (32, 64, 56, 56, 128, 3, 3, 2, 2, 1, 1)
     assert not fused(FWD, strided)["taken"]             # overlapping windows, not at stride 1
     p = fused(DX, strided)
@@ -88,3 +90,51 @@ def test_patch_slots_are_free_and_ready(taps):
         assert copied < cg * taps // 4, (taps, cg)
         if cg > 2:                                   # one copy per stage at most
             assert copied > -(-(cg - 2) * taps // 4)
+
+
+def test_weight_gradient_chunks_fit_every_block():
+    """A chunk of RC output rows' source rows fits its patch slot wherever the chunk starts, and two
+    to sixteen k steps of eight quads of four columns cover it."""
+    rng = random.Random(12)
+    found = 0
+    while found < 60:
+        k = rng.choice([(2, 2), (3, 3), (3, 3), (5, 5), (7, 7), (1, 7), (5, 2), (1, 1)])
+        n, c, f = rng.randint(1, 40), rng.choice([1, 3, 13, 16, 64, 130]), rng.choice([6, 33, 64])
+        h, w = rng.randint(k[0], 90), rng.randint(k[1], 300)
+        sy, sx = rng.choice([1, 1, 2, 3]), rng.choice([1, 1, 2])
+        shape = (n, c, h, w, f, k[0], k[1], sy, sx, rng.randint(0, k[0] - 1), rng.randint(0, k[1] - 1))
+        p = fused(DW, shape)
+        if not p["taken"]:
+            continue
+        found += 1
+        N, C, H, W, F, KH, KW, SY, SX, PY, PX = shape
+        OH, OW = (H + 2 * PY - KH) // SY + 1, (W + 2 * PX - KW) // SX + 1
+        rc, ns, sw = p["classes"], p["strips"], p["width"]
+        assert sw % 4 == 0 and ns * sw >= OW > (ns - 1) * sw, (shape, p)
+        channels = max((min(q + BLOCK, C * KH * KW) - 1) // (KH * KW) - q // (KH * KW) + 1
+                       for q in range(0, C * KH * KW, BLOCK))
+        assert channels * (64 * p["groups"] + 20) <= 6144 and p["groups"] <= 6, (shape, p)
+        ph, pw = (OH - 1) * SY + KH, (sw - 1) * SX + KW
+        assert 1 <= rc * sw // 4 <= 8 * 16, (shape, p)
+
+        def padded(v):
+            return v // OH * ph + v % OH * SY
+
+        rows = N * ns * OH
+        for v0 in range(0, rows, rc):
+            last = min(v0 + rc, rows) - 1
+            assert (padded(last) - padded(v0) + KH) * pw <= 64 * p["groups"], (shape, p, v0)
+
+
+@pytest.mark.parametrize("steps", range(2, 17))
+def test_weight_gradient_slots_are_free_and_ready(steps):
+    """Stage s takes k steps 2 s and 2 s + 1, step j chunk j // steps from patch slot (chunk % 2) and
+    table slot (chunk % 4). Chunk c >= 2 is copied, and table c + 2 built, during the first stage
+    that starts past chunk c - 2's last step; chunk c's quads are looked up when dY is loaded, two
+    stages before their own."""
+    for c in range(2, 40):
+        copied = -(-(c - 1) * steps // 2)
+        assert 2 * copied >= (c - 1) * steps and copied < c * steps // 2, (steps, c)
+        if c >= 4:  # tables 0 .. 3 are built before the first stage
+            built = -(-(c - 3) * steps // 2)
+            assert built + 1 <= c * steps // 2 - 2, (steps, c)

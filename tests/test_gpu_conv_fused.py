@@ -1,14 +1,14 @@
-"""GPU parity of the fused convolution kernels (forward pass and input gradient) with the oracle,
+"""GPU parity of the fused convolution kernels (forward pass and both gradients) with the oracle,
 bit for bit, at the sizes where they can go wrong: blocks and patches that span images and column
 strips, tiles cut by the last position and channel, channel counts off a group of 16, parts along
 k, residue classes of a strided input gradient (some without taps), kernels larger than the image,
-scales past one normal float, NaN and infinities."""
+output rows that are not whole quads, scales past one normal float, NaN and infinities."""
 import numpy as np
 import pytest
 
 from gpu_util import note
 from oracle import oracle as O
-from test_conv_fused_plan import DX, FWD, fused
+from test_conv_fused_plan import DW, DX, FWD, fused
 from test_gpu_conv import RC, _oracle, _run_algo
 
 pytestmark = pytest.mark.gpu
@@ -31,6 +31,10 @@ SHAPES = [
     (1, 16, 3, 3, 16, 3, 3, 1, 1, 3, 3),        # padding wider than the image
     (2, 16, 3, 4, 20, 9, 9, 1, 1, 4, 4),        # kernel larger than the image
     (5, 16, 7, 7, 16, 4, 4, 1, 2, 3, 0),
+    (40, 3, 28, 28, 6, 5, 5, 1, 1, 2, 2),       # weight gradient: one of four wavefronts has positions
+    (2, 30, 56, 56, 40, 3, 3, 1, 1, 1, 1),      # three position tiles, the last ragged
+    (1, 3, 50, 300, 20, 3, 3, 2, 2, 1, 1),      # column stride 2, strips
+    (9, 20, 24, 22, 33, 3, 3, 3, 1, 0, 0),      # row stride 3, rows of 20 columns
 ]
 
 
@@ -45,10 +49,10 @@ def _inputs(shape, seed):
 
 
 def _check(torch, shape, S, x, w, dy):
-    for kind, a in (("fwd", x), ("dX", dy)):
+    for kind, a, b in (("fwd", x, w), ("dX", dy, w), ("dW", dy, x)):
         note("fused conv", kind, shape, "S=%d" % S)
-        got = _run_algo(torch, kind, a, w, shape, S, RC.ALGO_GEMM).view(np.uint32).ravel()
-        assert np.array_equal(got, _oracle(kind, a, w, shape, S).view(np.uint32).ravel()), (kind, shape, S)
+        got = _run_algo(torch, kind, a, b, shape, S, RC.ALGO_GEMM).view(np.uint32).ravel()
+        assert np.array_equal(got, _oracle(kind, a, b, shape, S).view(np.uint32).ravel()), (kind, shape, S)
 
 
 @pytest.mark.parametrize("S", [1, 2, 3])
@@ -66,13 +70,16 @@ def test_shapes_cover_the_routes():
         assert any(not f["patch"] for f in mine)
         assert any(f["strips"] > 1 for f in mine)
         assert {f["tf"] for f in mine} == {1, 2}
+    mine = [(s, f) for s in SHAPES for f in [fused(DW, s)] if f["taken"]]
+    assert len(mine) >= 10 and any(f["strips"] > 1 for _, f in mine) and {f["tf"] for _, f in mine} == {1, 2}
+    assert {s[8] for s, _ in mine} == {1, 2} and any((s[3] + 2 * s[10] - s[6]) // s[8] % 4 != 3 for s, _ in mine)
 
 
 @pytest.mark.parametrize("what", ["tiny", "huge", "nonfinite"])
 def test_fused_slow_rounding(torch_gpu, what):
     """Rows whose scale is not one normal float (maxima below 2^-100 or near 2^127) and values
     that are not finite leave the one-multiply-add rounding."""
-    for shape in (SHAPES[1], SHAPES[9], SHAPES[10]):
+    for shape in (SHAPES[1], SHAPES[9], SHAPES[10], SHAPES[17]):
         x, w, dy = _inputs(shape, 77)
         rng = np.random.default_rng(5)
         for t in (x, dy):
