@@ -1,22 +1,39 @@
 // Exact, order-independent float32 sums (bias gradients, loss means) and the non-finite
 // scan, for the layers built on the reproducible GEMM.
 //
-// Accumulation: every thread owns a 10-limb superaccumulator in LDS (limb l of thread t at
-// acc[l][t], radix 2^32, limb l weighing 2^(32 l - 149)). A finite float is one wide term
-// v < 2^55 at limb idx = (biased exponent - 1) / 32 (repro_sum::wide_term), added with a
-// single 64-bit LDS read-modify-write; nobody else touches that address, so no atomics are
-// needed. At most 252 wide adds land between carry resolutions, which keeps every limb below
-// 2^32 + 252 * 2^55 < 2^63. Threads, waves, blocks and chunks are then merged by integer
-// addition of normalised limbs (exact and associative), and one thread per output divides
-// exactly (for a mean) and rounds once (repro_sum::finalize).
+// Accumulation: a thread adds its values in binary64 while that is exact. Values whose magnitudes
+// lie in [2^l, 2^(h+1)) are integers times 2^(l-23), so n of them sum to at most n 2^(h+1-l+23) such
+// units, and every partial sum is exact while h - l + ceil(log2 n) <= 29: a thread keeps the largest
+// magnitude and the smallest non-zero one of what its binary64 sum holds (16 values at a time), and
+// when the next 16 would break the bound it moves the sum into its superaccumulator and starts
+// again; 16 values that break it by themselves go into the superaccumulator one by one. N(0, 1)
+// data never does either within a thread's share. A value costs about five vector instructions
+// (widening, addition, the two bounds) instead of a read-modify-write of LDS.
+//
+// The superaccumulator is exact for every float: 10 limbs per thread in LDS (limb l of thread t at
+// acc[l][t], radix 2^32, limb l weighing 2^(32 l - 149)), cleared when a thread first needs it. A
+// finite float is one wide term v < 2^55 at limb idx = (biased exponent - 1) / 32
+// (repro_sum::wide_term); at most 252 wide adds land between carry resolutions, which keeps every
+// limb below 2^32 + 252 * 2^55 < 2^63. Threads, waves, blocks and chunks are merged by integer
+// addition of normalised limbs (exact and associative), and one thread per output divides exactly
+// (for a mean) and rounds once (repro_sum::finalize). A wave whose lanes' sums still satisfy the
+// bound together adds them in binary64 and, where the output has no other chunk and no division,
+// rounds that one exact sum.
 //
 // Kernels by layout of x = [A][B][C]:
 //   C == 1   columns: a 256-thread block covers 64 outputs x 4 row phases; a wave reads
 //            64 consecutive floats of one row (bias gradient of a Linear layer).
-//   C >  1   segments: one wave per (output, chunk) walks contiguous runs of C floats
-//            (conv bias gradient, loss mean, row sums).
+//   C >  1   segments: one wave per (output, chunk) walks the output's values, runs of C contiguous
+//            floats (conv bias gradient, loss mean, row sums), by 16-byte loads where they allow it.
 // With more than one chunk per output, the chunks' limbs go to the workspace and a third
 // kernel merges and rounds them.
+//
+// Measured on MI355X against the LDS accumulation of every value (us, whole sum): 256 x 64 x 3136
+// 87 -> 37 (5.6 TB/s), 8192 x 4096 rows 45 -> 25 (5.3 TB/s) and columns 56 -> 28, 16384 rows of 1024
+// 34 -> 14.5, 65536 rows of 128 86 -> 27, 1000 x 33 x 7 27 -> 5, one sum of 2^24 values 38 -> 23 (the
+// merge of its 2048 chunks is one block's). The large ones run at the rate of a copy's reads; small
+// ones are two launches.
+#include "rg_fastdiv.h"
 #include "rg_internal.h"
 #include "repro_sum.h"
 #include "repro_sum_math.h"
@@ -30,13 +47,13 @@ namespace {
 using repro_sum::LIMBS;
 
 constexpr int SUM_THREADS = 256;
-constexpr int GROUP = 4;          // loads issued together per thread
+constexpr int BATCH = 16;         // values a thread loads and adds together
 constexpr int FLUSH_AT = 252;     // wide adds per limb between carry resolutions
 constexpr size_t SUM_ALIGN = 256;
 
 size_t align_up(size_t x) { return (x + SUM_ALIGN - 1) / SUM_ALIGN * SUM_ALIGN; }
 
-// Thread-private accumulator in LDS: limb l at p[l * SUM_THREADS].
+// Thread-private superaccumulator in LDS: limb l at p[l * SUM_THREADS].
 struct LdsAcc {
     int64_t* p;
 
@@ -54,6 +71,30 @@ struct LdsAcc {
         }
         p[idx * SUM_THREADS] += neg ? -(int64_t)v : (int64_t)v;
     }
+    // An exact sum of floats held in binary64 (a multiple of 2^-149 below 2^159): its 53-bit
+    // significand, shifted to a limb boundary, is three 32-bit terms.
+    __device__ void add_double(double x, int& nonfinite) {
+        const uint64_t b = (uint64_t)__double_as_longlong(x);
+        const int e = (int)(b >> 52) & 0x7FF;
+        if (e == 0x7FF) {
+            nonfinite = 1;
+            return;
+        }
+        if (e == 0) return;  // zero: the smallest non-zero sum, 2^-149, is a normal binary64
+        uint64_t m = (b & 0xFFFFFFFFFFFFFull) | 0x10000000000000ull;
+        int sh = e - 1075 + 149;  // |x| = m 2^(sh - 149)
+        if (sh < 0) {  // (the bits shifted out are zeros)
+            m >>= -sh;
+            sh = 0;
+        }
+        const int idx = sh >> 5, s = sh & 31;
+        const int64_t t0 = (int64_t)(uint32_t)(m << s);
+        const int64_t t1 = (int64_t)(uint32_t)(m >> (32 - s)), t2 = s ? (int64_t)(m >> (64 - s)) : 0;
+        const int64_t sign = (int64_t)b >> 63;  // 0 or -1
+        p[idx * SUM_THREADS] += (t0 ^ sign) - sign;
+        p[(idx + 1) * SUM_THREADS] += (t1 ^ sign) - sign;
+        p[(idx + 2) * SUM_THREADS] += (t2 ^ sign) - sign;
+    }
     // Carries: limbs 0..LIMBS-2 into [0, 2^32), the top limb keeps the sign.
     __device__ void carry() {
         int64_t c = 0;
@@ -69,19 +110,95 @@ struct LdsAcc {
     }
 };
 
-// Writes one output's merged limbs: rounds them when this is the only chunk, else stores them
-// as chunk `chunk` of output b.
-__device__ void emit(const int64_t* limbs, int stride, int nonfinite, int b, int B, int chunk,
-                     int chunks, uint32_t divisor, float* out, int64_t* part, int* part_nf) {
-    if (chunks == 1) {
-        out[b] = repro_sum::finalize(limbs, stride, divisor, nonfinite);
-    } else {
-#pragma unroll
-        for (int l = 0; l < LIMBS; ++l)
-            part[((size_t)chunk * LIMBS + l) * B + b] = limbs[l * stride];
-        part_nf[(size_t)chunk * B + b] = nonfinite;
-    }
+// ceil(log2(n)) for n >= 1.
+__device__ __forceinline__ int log2_up(uint32_t n) { return 32 - __clz((int)(n - 1)); }
+
+// Whether n values with largest magnitude `top` and smallest non-zero one `low` sum exactly in
+// binary64 in any order: h - l + ceil(log2 n) <= 29. low is kept as 2 * bits - 1 without the sign
+// (zeros map to the largest key, so they never are the smallest); a subnormal counts as the smallest
+// normal exponent, whose last bit is its unit. An infinity fails the bound.
+__device__ __forceinline__ bool sums_exactly(float top, uint32_t low, int log2n) {
+    const int h = (int)(__float_as_uint(top) >> 23), l = max(1, (int)(low >> 24));
+    return max(h, 1) - l + log2n <= 29;
 }
+
+// A thread's sum: binary64 while exact, the superaccumulator otherwise.
+struct ThreadSum {
+    LdsAcc limbs;
+    double acc0 = 0.0, acc1 = 0.0;
+    float top = 0.0f;            // of what acc0 + acc1 hold
+    uint32_t low = 0xFFFFFFFFu;
+    uint32_t count = 0;
+    int since = 0;               // additions to the limbs since their carries
+    bool used = false;           // the limbs hold something (and were cleared)
+    int nonfinite = 0;
+
+    __device__ void spill() {    // binary64 -> limbs
+        if (!used) {
+            limbs.clear();
+            used = true;
+        }
+        limbs.add_double(acc0 + acc1, nonfinite);
+        ++since;
+        acc0 = acc1 = 0.0;
+        top = 0.0f;
+        low = 0xFFFFFFFFu;
+        count = 0;
+    }
+    template <int N>
+    __device__ __forceinline__ void add(const float (&v)[N]) {
+        // A NaN is in neither bound; it makes the binary64 sum a NaN, which spill() and the final
+        // steps see.
+        float m = top;
+        uint32_t k = low;
+#pragma unroll
+        for (int i = 0; i < N; ++i) m = fmaxf(m, __builtin_fabsf(v[i]));
+#pragma unroll
+        for (int i = 0; i < N; ++i) k = min(k, 2u * __float_as_uint(v[i]) - 1u);
+        if (__builtin_expect(!sums_exactly(m, k, log2_up(count + N)), 0)) {
+            spill();
+#pragma unroll
+            for (int i = 0; i < N; ++i) top = fmaxf(top, __builtin_fabsf(v[i]));
+#pragma unroll
+            for (int i = 0; i < N; ++i) low = min(low, 2u * __float_as_uint(v[i]) - 1u);
+            if (!sums_exactly(top, low, log2_up(N))) {
+#pragma unroll 1
+                for (int i = 0; i < N; ++i) {
+                    float x = v[0];
+#pragma unroll
+                    for (int j = 1; j < N; ++j) x = i == j ? v[j] : x;
+                    limbs.add(x, nonfinite);
+                }
+                since += N;
+                top = 0.0f;
+                low = 0xFFFFFFFFu;
+                if (since >= FLUSH_AT - BATCH) {
+                    limbs.carry();
+                    since = 0;
+                }
+                return;
+            }
+            if (since >= FLUSH_AT - BATCH) {
+                limbs.carry();
+                since = 0;
+            }
+        } else {
+            top = m;
+            low = k;
+        }
+        count += N;
+#pragma unroll
+        for (int i = 0; i < N; i += 2) {
+            acc0 += (double)v[i];
+            if (i + 1 < N) acc1 += (double)v[i + 1];
+        }
+    }
+    // Everything into normalised limbs.
+    __device__ void finish() {
+        spill();
+        limbs.carry();
+    }
+};
 
 // C == 1. Block = 64 outputs (lanes) x 4 row phases (waves); chunk = blockIdx.y covers rows
 // [a0, a1), phase w takes rows a0 + w, a0 + w + 4, ...
@@ -96,129 +213,179 @@ sum_columns(const float* __restrict__ x, int A, int B, int rows_per_chunk, int c
     const int chunk = blockIdx.y;
     const int a0 = chunk * rows_per_chunk;
     const int a1 = min(A, a0 + rows_per_chunk);
-    LdsAcc acc_t{acc + t};
-    acc_t.clear();
-    int nf = 0;
+    ThreadSum sum{LdsAcc{acc + t}};
     if (b < B) {
-        int since = 0;
-        for (int a = a0 + phase; a < a1; a += 4 * GROUP) {
-            float v[GROUP];
+        for (int a = a0 + phase; a < a1; a += 4 * BATCH) {
+            float v[BATCH];
 #pragma unroll
-            for (int g = 0; g < GROUP; ++g) {
+            for (int g = 0; g < BATCH; ++g) {
                 const int r = a + 4 * g;
                 v[g] = r < a1 ? x[(size_t)r * B + b] : 0.0f;
             }
-#pragma unroll
-            for (int g = 0; g < GROUP; ++g) acc_t.add(v[g], nf);
-            since += GROUP;
-            if (since >= FLUSH_AT) {
-                acc_t.carry();
-                since = 0;
-            }
+            sum.add<BATCH>(v);
         }
     }
-    acc_t.carry();
-    nf_sh[t] = nf;
+    sum.finish();
+    nf_sh[t] = sum.nonfinite;
     __syncthreads();
-    if (phase == 0 && b < B) {
+    // The four phases' limbs: thread t adds limb (t >> 6) + 4 i of output t & 63.
 #pragma unroll
-        for (int l = 0; l < LIMBS; ++l) {
-            int64_t s = 0;
+    for (int l = phase; l < LIMBS; l += 4) {
+        int64_t s = 0;
 #pragma unroll
-            for (int w = 0; w < 4; ++w) s += acc[l * SUM_THREADS + t + 64 * w];
-            acc[l * SUM_THREADS + t] = s;
+        for (int w = 0; w < 4; ++w) s += acc[l * SUM_THREADS + col + 64 * w];
+        if (chunks > 1) {
+            if (b < B) part[((size_t)chunk * LIMBS + l) * B + b] = s;
+        } else {
+            acc[l * SUM_THREADS + col] = s;  // (only this thread reads the four)
         }
-        const int nfb = nf_sh[t] | nf_sh[t + 64] | nf_sh[t + 128] | nf_sh[t + 192];
-        emit(acc + t, SUM_THREADS, nfb, b, B, chunk, chunks, divisor, out, part, part_nf);
     }
+    const int nf = nf_sh[col] | nf_sh[col + 64] | nf_sh[col + 128] | nf_sh[col + 192];
+    if (chunks > 1) {
+        if (phase == 0 && b < B) part_nf[(size_t)chunk * B + b] = nf;
+        return;
+    }
+    __syncthreads();
+    if (phase == 0 && b < B) out[b] = repro_sum::finalize(acc + col, SUM_THREADS, divisor, nf);
 }
 
 // C > 1. Wave w of block x handles item 4 x + w of the B * chunks (output, chunk) items,
 // output b = item / chunks, chunk item % chunks: summands [i0, i1) of the A*C values of b, in
-// order a-major, walked as contiguous runs of x. Every wave of a block has work when
-// B * chunks fills the grid, however small B is.
+// order a-major (VEC: in fours, C a multiple of four and x 16-byte aligned). Every wave of a block
+// has work when B * chunks fills the grid, however small B is.
+template <bool VEC>
 __global__ void __launch_bounds__(SUM_THREADS)
-sum_segments(const float* __restrict__ x, int A, int B, int C, int chunks, uint32_t divisor,
+sum_segments(const float* __restrict__ x, int A, int B, int C, FastDiv dC, int chunks, uint32_t divisor,
              float* __restrict__ out, int64_t* __restrict__ part, int* __restrict__ part_nf) {
     __shared__ int64_t acc[LIMBS * SUM_THREADS];
     __shared__ int64_t merged[4][LIMBS];
-    __shared__ int nf_sh[SUM_THREADS];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const long long item = (long long)blockIdx.x * 4 + w;
-    const int b = item < (long long)B * chunks ? (int)(item / chunks) : B;  // B: no work
-    const int chunk = b < B ? (int)(item - (long long)b * chunks) : 0;
-    LdsAcc acc_t{acc + t};
-    acc_t.clear();
-    int nf = 0;
-    if (b < B) {
-        const long long count = (long long)A * C;
-        const long long i0 = count * chunk / chunks, i1 = count * (chunk + 1) / chunks;
-        int a = (int)(i0 / C);
-        int c = (int)(i0 - (long long)a * C);
-        long long left = i1 - i0;
-        int since = 0;
-        while (left > 0) {
-            const int len = (int)std::min<long long>(C - c, left);
-            const float* p = x + ((size_t)a * B + b) * C + c;
-            for (int j = lane; j < len; j += 64 * GROUP) {
-                float v[GROUP];
-#pragma unroll
-                for (int g = 0; g < GROUP; ++g) {
-                    const int k = j + 64 * g;
-                    v[g] = k < len ? p[k] : 0.0f;
-                }
-#pragma unroll
-                for (int g = 0; g < GROUP; ++g) acc_t.add(v[g], nf);
-                since += GROUP;
-                if (since >= FLUSH_AT) {
-                    acc_t.carry();
-                    since = 0;
-                }
-            }
-            left -= len;
-            ++a;
-            c = 0;
+    if (item >= (long long)B * chunks) return;  // (no block barrier below)
+    const int b = (int)(item / chunks), chunk = (int)(item - (long long)b * chunks);
+    ThreadSum sum{LdsAcc{acc + t}};
+    constexpr int V = VEC ? 4 : 1;
+    const long long units = (long long)A * C / V;
+    const uint32_t u0 = (uint32_t)(units * chunk / chunks), u1 = (uint32_t)(units * (chunk + 1) / chunks);
+    auto load = [&](uint32_t ug, float* v) {
+        const uint32_t i = min(ug, u1 - 1) * V;
+        const uint32_t a = fdiv(i, dC);
+        const float* p = x + ((size_t)a * B + b) * C + (i - a * (uint32_t)C);
+        if (VEC) {
+            float4 q = *reinterpret_cast<const float4*>(p);
+            if (ug >= u1) q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            v[0] = q.x;
+            v[1] = q.y;
+            v[2] = q.z;
+            v[3] = q.w;
+        } else {
+            v[0] = ug < u1 ? *p : 0.0f;
         }
+    };
+    constexpr int G = BATCH / V;  // loads of a batch; a short rest (or row) goes one load at a time
+    uint32_t u = u0 + lane;
+    for (; u - lane + 64 * (G / 4) < u1; u += 64 * G) {
+        float v[BATCH];
+#pragma unroll
+        for (int g = 0; g < G; ++g) load(u + 64 * g, v + V * g);
+        sum.add<BATCH>(v);
     }
-    acc_t.carry();
-    nf_sh[t] = nf;
-    __syncthreads();
-    if (b < B && lane < LIMBS) {
-        int64_t s = 0;
-        for (int j = 0; j < 64; ++j) s += acc[lane * SUM_THREADS + 64 * w + j];  // < 2^38
-        merged[w][lane] = s;
+    for (; u - lane < u1; u += 64) {
+        float v[V];
+        load(u, v);
+        sum.add<V>(v);
     }
-    if (b < B && lane == LIMBS) {
-        int any = 0;
-        for (int j = 0; j < 64; ++j) any |= nf_sh[64 * w + j];
-        nf_sh[64 * w] = any;  // read back by lane 0 of this wave after the barrier
+    // The wave's lanes in binary64 where that is exact (a NaN or an infinity makes the sum one).
+    float top = sum.top;
+    uint32_t low = sum.low;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        top = fmaxf(top, __shfl_xor(top, off, 64));
+        low = min(low, (uint32_t)__shfl_xor((int)low, off, 64));
     }
-    __syncthreads();
-    if (b < B && lane == 0)
-        emit(merged[w], 1, nf_sh[64 * w], b, B, chunk, chunks, divisor, out, part, part_nf);
+    const uint32_t total = (u1 - u0) * V + 64u * BATCH;  // at least what the lanes added
+    const bool exact = __ballot(sum.used) == 0 && sums_exactly(top, low, log2_up(total));
+    if (exact && chunks == 1 && divisor == 1) {
+        double s = sum.acc0 + sum.acc1;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        if (lane == 0) {
+            // A zero sum is +0.0; a NaN among the values gives the NaN of repro_sum::finalize.
+            const bool nan = !(__builtin_fabs(s) < __builtin_inf());
+            out[b] = nan ? __uint_as_float(0x7FC00000u) : (s == 0.0 ? 0.0f : (float)s);
+        }
+        return;
+    }
+    sum.finish();
+    const int nf = __ballot(sum.nonfinite != 0) != 0;
+    // Limb l of the wave: four lanes add 16 threads' limbs each. (A wave's LDS operations are in
+    // order, and only this wave's threads' limbs are read.)
+    __builtin_amdgcn_wave_barrier();
+    int64_t s = 0;
+    if (lane < 4 * LIMBS) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s += acc[(lane >> 2) * SUM_THREADS + 64 * w + 16 * (lane & 3) + j];  // < 2^38
+    }
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    if (chunks > 1) {
+        if (lane < 4 * LIMBS && (lane & 3) == 0) part[((size_t)chunk * LIMBS + (lane >> 2)) * B + b] = s;
+        if (lane == 0) part_nf[(size_t)chunk * B + b] = nf;
+        return;
+    }
+    if (lane < 4 * LIMBS && (lane & 3) == 0) merged[w][lane >> 2] = s;
+    __builtin_amdgcn_wave_barrier();
+    if (lane == 0) out[b] = repro_sum::finalize(merged[w], 1, divisor, nf);
 }
 
-// Merges the chunks of each output and rounds once. Few chunks: a thread per output adds
-// them; many: a block per output, thread t adding chunks t, t + 256, ... and the block
-// reducing its threads' sums. Either way the normalised limbs (each < 2^32) of at most 65535
-// chunks sum below 2^48 in int64.
-constexpr int MERGE_BLOCK_FROM = 32;
+// Merges the chunks of each output and rounds once. Few chunks: 32 outputs a block, eight threads
+// each (consecutive threads take consecutive outputs; thread s adds chunks s, s + 8, ...); many: a
+// block per output, thread t adding chunks t, t + 256, ... Either way the block adds its threads'
+// sums in LDS; the normalised limbs (each < 2^32) of at most 65535 chunks sum below 2^48 in int64.
+constexpr int MERGE_BLOCK_FROM = 64;
 
 __global__ void __launch_bounds__(SUM_THREADS)
-sum_merge_threads(const int64_t* __restrict__ part, const int* __restrict__ part_nf, int B,
-                  int chunks, uint32_t divisor, float* __restrict__ out) {
-    const int b = blockIdx.x * SUM_THREADS + threadIdx.x;
-    if (b >= B) return;
+sum_merge_groups(const int64_t* __restrict__ part, const int* __restrict__ part_nf, int B,
+                 int chunks, uint32_t divisor, float* __restrict__ out) {
+    __shared__ int64_t red[LIMBS][SUM_THREADS];
+    __shared__ int nf_sh[SUM_THREADS];
+    const int t = threadIdx.x, o = t & 31, sub = t >> 5;
+    const int b = blockIdx.x * 32 + o;
     int64_t tot[LIMBS];
 #pragma unroll
     for (int l = 0; l < LIMBS; ++l) tot[l] = 0;
     int nf = 0;
-    for (int k = 0; k < chunks; ++k) {
+    if (b < B) {
+        for (int k = sub; k < chunks; k += 16) {  // two chunks' loads together
+            const int k2 = k + 8 < chunks ? k + 8 : k;
+            int64_t v[2][LIMBS];
 #pragma unroll
-        for (int l = 0; l < LIMBS; ++l) tot[l] += part[((size_t)k * LIMBS + l) * B + b];
-        nf |= part_nf[(size_t)k * B + b];
+            for (int l = 0; l < LIMBS; ++l) {
+                v[0][l] = part[((size_t)k * LIMBS + l) * B + b];
+                v[1][l] = part[((size_t)k2 * LIMBS + l) * B + b];
+            }
+            nf |= part_nf[(size_t)k * B + b] | part_nf[(size_t)k2 * B + b];
+#pragma unroll
+            for (int l = 0; l < LIMBS; ++l) tot[l] += v[0][l] + (k2 == k ? 0 : v[1][l]);
+        }
     }
-    out[b] = repro_sum::finalize(tot, 1, divisor, nf);
+#pragma unroll
+    for (int l = 0; l < LIMBS; ++l) red[l][t] = tot[l];
+    nf_sh[t] = nf;
+    __syncthreads();
+    // Thread (o, sub) adds limbs sub and sub + 8 of output o; its own column is no other's.
+    for (int l = sub; l < LIMBS; l += 8) {
+        int64_t s = 0;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) s += red[l][o + 32 * g];
+        red[l][o] = s;
+    }
+    __syncthreads();
+    if (sub == 0 && b < B) {
+#pragma unroll
+        for (int g = 1; g < 8; ++g) nf |= nf_sh[o + 32 * g];
+        out[b] = repro_sum::finalize(&red[0][o], SUM_THREADS, divisor, nf);
+    }
 }
 
 __global__ void __launch_bounds__(SUM_THREADS)
@@ -385,14 +552,15 @@ int rg_sum_fp32_ws(const float* x, float* out, int A, int B, int C, const rg_sum
     } else {
         const long long items = (long long)B * L.chunks;
         if ((items + 3) / 4 > INT_MAX) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(rg::sum_segments, dim3((unsigned)((items + 3) / 4)), dim3(rg::SUM_THREADS),
-                           0, stream, x, A, B, C, L.chunks, divisor, out, part, part_nf);
+        const bool vec = C % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+        const auto segments = vec ? rg::sum_segments<true> : rg::sum_segments<false>;
+        hipLaunchKernelGGL(segments, dim3((unsigned)((items + 3) / 4)), dim3(rg::SUM_THREADS), 0, stream,
+                           x, A, B, C, rg::make_fastdiv((uint32_t)C), L.chunks, divisor, out, part, part_nf);
     }
     if (L.chunks > 1) {
         if (L.chunks < rg::MERGE_BLOCK_FROM)
-            hipLaunchKernelGGL(rg::sum_merge_threads, dim3((B + rg::SUM_THREADS - 1) / rg::SUM_THREADS),
-                               dim3(rg::SUM_THREADS), 0, stream, part, part_nf, B, L.chunks,
-                               divisor, out);
+            hipLaunchKernelGGL(rg::sum_merge_groups, dim3((B + 31) / 32), dim3(rg::SUM_THREADS), 0, stream,
+                               part, part_nf, B, L.chunks, divisor, out);
         else
             hipLaunchKernelGGL(rg::sum_merge, dim3((unsigned)B), dim3(rg::SUM_THREADS), 0, stream,
                                part, part_nf, B, L.chunks, divisor, out);

@@ -101,11 +101,15 @@ RG_HD inline float finalize(const int64_t* acc, int stride, uint32_t divisor, in
     constexpr int D = LIMBS + 2;                // digits of |value| * 2^64
     uint32_t q[D];
     uint64_t rem = 0;
-    for (int i = D - 1; i >= 0; --i) {
-        const uint64_t digit = i >= 2 ? (uint64_t)(uint32_t)t[i - 2] : 0u;
-        const uint64_t cur = (rem << 32) | digit;   // < divisor * 2^32 <= 2^63
-        q[i] = (uint32_t)(cur / divisor);
-        rem = cur % divisor;
+    if (divisor == 1) {  // a sum: no division (twelve long ones on a GPU)
+        for (int i = D - 1; i >= 0; --i) q[i] = i >= 2 ? (uint32_t)t[i - 2] : 0u;
+    } else {
+        for (int i = D - 1; i >= 0; --i) {
+            const uint64_t digit = i >= 2 ? (uint64_t)(uint32_t)t[i - 2] : 0u;
+            const uint64_t cur = (rem << 32) | digit;   // < divisor * 2^32 <= 2^63
+            q[i] = (uint32_t)(cur / divisor);
+            rem = cur % divisor;
+        }
     }
     int top = D - 1;
     while (top >= 0 && q[top] == 0) --top;
