@@ -85,7 +85,7 @@ int blocks_per_cu(int ti, int tj, int S) {
     return std::max(1, std::min(2, (160 * 1024) / lds_bytes));
 }
 
-// Tile rows per group of the contraction's block order (block_tile): the power of two that
+// Tile rows per group of the contraction's block order (block_of): the power of two that
 // keeps the digit panels touched by one XCD's run of `chunk` consecutive tiles (row panels of
 // 64 ti rows, column panels of 64 tj columns) fewest. A run from the start of a group covers
 // that group column by column, then the next group.
@@ -725,10 +725,11 @@ int rg_test_block_order(int M, int N, int K, const rg_config* cfg, int is_gfx950
     const long long total = (long long)tiles_m * tiles_n * L.split * L.batch;
     *blocks = total;
     if (!coords || capacity < 4 * total) return hipSuccess;
+    const rg::BlockOrder order = rg::make_block_order(tiles_m, tiles_n, L.split, L.batch, L.xcd_chunk,
+                                                      L.group_m, L.Kp / rg::STEP_K);
     for (long long i = 0; i < total; ++i) {
-        int item, part, tm, tn;
-        rg::block_tile(rg::xcd_order((int)i, (int)total, L.xcd_chunk), tiles_m, tiles_n, L.split,
-                       L.group_m, &item, &part, &tm, &tn);
+        int item, part, tm, tn, s0, s1;
+        rg::block_of(order, (int)i, &item, &part, &tm, &tn, &s0, &s1);
         coords[4 * i] = item;
         coords[4 * i + 1] = part;
         coords[4 * i + 2] = tm;

@@ -41,8 +41,8 @@ template <int S, int WTI, int WTJ, int WGM, int WGN>
 __global__ void __launch_bounds__(64 * WGM * WGN, (contract_waves_per_simd<S, WTI, WTJ, WGM, WGN>()))
 contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
               const int* __restrict__ eA, const int* __restrict__ eB, float* __restrict__ C,
-              int64_t* __restrict__ partial, int M, int N, int Kp, int split, int tiles_n,
-              int Mp, int Np, long long ldc, long long c_item, int xcd_chunk, int group_m) {
+              int64_t* __restrict__ partial, int M, int N, int Kp, int Mp, int Np, long long ldc,
+              long long c_item, BlockOrder order) {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer resources exist only in the device pass
     constexpr int L = 2 * S - 1;
     constexpr int NW = WGM * WGN;                  // wavefronts per block
@@ -65,14 +65,10 @@ contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
     // The grid is (tiles, split, batch); which tile, part and item this block computes follows
-    // the XCD-aware block order (xcd_order, block_tile), a bijection of the grid's blocks.
-    int tm, tn, part, item;
-    {
-        const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-        const int total = gridDim.x * gridDim.y * gridDim.z;
-        block_tile(xcd_order(lin, total, xcd_chunk), gridDim.x / tiles_n, tiles_n, split, group_m,
-                   &item, &part, &tm, &tn);
-    }
+    // the XCD-aware block order (block_of), a bijection of the grid's blocks.
+    int tm, tn, part, item, s0, s1;
+    block_of(order, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), &item, &part, &tm, &tn,
+             &s0, &s1);
     // Item of a batch: its digit panels, exponents, output and partials follow the previous
     // item's (item 0 for a single GEMM).
     QA += (size_t)item * Mp * Kp * S;
@@ -80,11 +76,8 @@ contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
     eA += (size_t)item * Mp;
     eB += (size_t)item * Np;
     if (C != nullptr) C += (size_t)item * c_item;
-    if (partial != nullptr) partial += (size_t)item * split * M * N;
-    const int nsteps = Kp / STEP_K;
-    const int s0 = (int)((long long)nsteps * part / split);
-    const int s1 = (int)((long long)nsteps * (part + 1) / split);
-    const size_t row_stride = (size_t)(Kp / PANEL_K) * S * (PANEL_BYTES / 16);  // in v4i
+    if (partial != nullptr) partial += (size_t)item * order.split * M * N;
+    const size_t row_bytes = (size_t)(uint32_t)Kp * (uint32_t)(S * PANEL_ROWS);  // of a 32-row panel
 
     // One buffer resource per panel this wavefront copies: base = the panel at stage s0,
     // range = this part's stages, so every offset is 32-bit whatever K is and an offset out
@@ -94,21 +87,19 @@ contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
     const uint32_t part_bytes = (uint32_t)(s1 - s0) * step_bytes;
     const bool copier = wave < CW;
     __amdgpu_buffer_rsrc_t rsrc[PW];
+    {
+        const int8_t* a0 = QA + (size_t)(uint32_t)(tm * (BM / PANEL_ROWS)) * row_bytes + (size_t)(uint32_t)s0 * step_bytes;
+        const int8_t* b0 = QB + (size_t)(uint32_t)(tn * (BN / PANEL_ROWS)) * row_bytes + (size_t)(uint32_t)s0 * step_bytes;
 #pragma unroll
-    for (int i = 0; i < PW; ++i) {
-        // (non-copying wavefronts never use rsrc)
-        const int pi = CW == NW ? wave + NW * i : (copier ? wave + CW * i : 0);
-        const int8_t* base;
-        if (pi < PA) {
-            const int rl = pi / (2 * S), o = pi % (2 * S);
-            base = QA + ((size_t)(tm * (BM / PANEL_ROWS) + rl) * row_stride + (size_t)o * (PANEL_BYTES / 16)) * 16;
-        } else {
-            const int pb = pi - PA;
-            const int cl = pb / (2 * S), o = pb % (2 * S);
-            base = QB + ((size_t)(tn * (BN / PANEL_ROWS) + cl) * row_stride + (size_t)o * (PANEL_BYTES / 16)) * 16;
+        for (int i = 0; i < PW; ++i) {
+            // (non-copying wavefronts never use rsrc)
+            const int pi = CW == NW ? wave + NW * i : (copier ? wave + CW * i : 0);
+            const bool of_a = pi < PA;
+            const int q = of_a ? pi : pi - PA;
+            const int rl = q / (2 * S), o = q - rl * (2 * S);
+            const int8_t* base = (of_a ? a0 : b0) + (size_t)(uint32_t)rl * row_bytes + (uint32_t)(o * PANEL_BYTES);
+            rsrc[i] = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)part_bytes, 0x00020000);
         }
-        base += (size_t)s0 * step_bytes;
-        rsrc[i] = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)part_bytes, 0x00020000);
     }
     const uint32_t voff = (uint32_t)lane * 16u;
 
@@ -864,11 +855,12 @@ static void launch_mfma_s(const Layout& L, const int8_t* qa, const int8_t* qb, c
                           hipStream_t stream) {
     const int tiles_m = L.Mp / (64 * L.ti), tiles_n = L.Np / (64 * L.tj);
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)L.split, (unsigned)L.batch);
+    const BlockOrder order =
+        make_block_order(tiles_m, tiles_n, L.split, L.batch, L.xcd_chunk, L.group_m, L.Kp / STEP_K);
     // Block tiles: 128x128 = 8 wavefronts of 64x32; 128x64 and 64x128 = 8 wavefronts of 32x32
     // (two per SIMD); 64x64 = 4 wavefronts of 32x32; 64x192 and 192x64 = 12 wavefronts of
     // 32x32 (three per SIMD).
-#define RG_CONTRACT_ARGS qa, qb, ea, eb, C, partial, L.M, L.N, L.Kp, L.split, tiles_n, L.Mp, L.Np, \
-                         out.ldc, out.c_item, L.xcd_chunk, L.group_m
+#define RG_CONTRACT_ARGS qa, qb, ea, eb, C, partial, L.M, L.N, L.Kp, L.Mp, L.Np, out.ldc, out.c_item, order
     // (The twelve-wavefront tiles exist for S = 3 only: their 48 stage panels split evenly over
     // 12 wavefronts; the planner never gives them to S < 3.)
     if constexpr (S == 3) {

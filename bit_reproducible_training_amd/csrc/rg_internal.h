@@ -117,19 +117,67 @@ __host__ __device__ inline int xcd_order(int lin, int total, int chunk) {
 // Logical block t -> (item, split part, tile row, tile column). Logical blocks run item by
 // item, part by part; within a part, tiles go through groups of `group_m` tile rows (the last
 // group may be shorter), column by column inside a group, so a run of consecutive tiles covers
-// a few row panels of op(A) and a few column panels of op(B).
-__host__ __device__ inline void block_tile(int t, int tiles_m, int tiles_n, int split,
-                                           int group_m, int* item, int* part, int* tm, int* tn) {
-    const int tiles = tiles_m * tiles_n;
-    const int ip = t / tiles, tile = t - ip * tiles;
-    *item = ip / split;
-    *part = ip - *item * split;
-    const int span = group_m * tiles_n;
-    const int g = tile / span, w = tile - g * span;
-    const int left = tiles_m - g * group_m;
-    const int rows = left < group_m ? left : group_m;
-    *tm = g * group_m + w % rows;
-    *tn = w / rows;
+// a few row panels of op(A) and a few column panels of op(B). The whole decode from the workgroup
+// id (xcd_order with chunk, then this), and the parts' shares of the `steps` pipeline stages, with
+// every divisor fixed on the host: by plain divisions (eleven of 32 bits, two of 64) they took most
+// of the 1000 scalar instructions, about 4000 cycles or 2 us, that a block of the contraction spent
+// before its first copy.
+struct BlockOrder {
+    int total;               // workgroups (tiles * split * batch)
+    int chunk, full, run;    // xcd_order: 0 or the run length; workgroups in full runs; the rest's run
+    int tiles, tiles_m, split, group_m;
+    int steps, extra;        // stages per part; the first `extra` parts take one more
+    FastDiv d_chunk, d_tiles, d_split, d_span, d_rows, d_last;
+};
+
+inline BlockOrder make_block_order(int tiles_m, int tiles_n, int split, int batch, int chunk, int group_m,
+                                   int nsteps) {
+    BlockOrder o;
+    o.tiles = tiles_m * tiles_n;
+    o.total = o.tiles * split * batch;
+    o.chunk = chunk;
+    o.full = chunk > 0 ? o.total / (8 * chunk) * (8 * chunk) : 0;
+    o.run = (o.total - o.full) / 8;
+    o.tiles_m = tiles_m;
+    o.split = split;
+    o.group_m = group_m;
+    o.steps = nsteps / split;
+    o.extra = nsteps % split;
+    const int last = tiles_m % group_m;  // tile rows of a shorter last group
+    o.d_chunk = make_fastdiv((uint32_t)(chunk > 0 ? chunk : 1));
+    o.d_tiles = make_fastdiv((uint32_t)o.tiles);
+    o.d_split = make_fastdiv((uint32_t)split);
+    o.d_span = make_fastdiv((uint32_t)group_m * (uint32_t)tiles_n);
+    o.d_rows = make_fastdiv((uint32_t)group_m);
+    o.d_last = make_fastdiv((uint32_t)(last > 0 ? last : group_m));
+    return o;
+}
+
+// The block that workgroup `lin` computes, and its part's stages [s0, s1).
+__host__ __device__ inline void block_of(const BlockOrder& o, int lin, int* item, int* part, int* tm,
+                                         int* tn, int* s0, int* s1) {
+    int t = lin;
+    if (o.chunk > 0) {  // xcd_order(lin, total, chunk)
+        const int xcd = lin & 7, loc = lin >> 3;
+        if (lin < o.full) {
+            const int q = (int)fdiv((uint32_t)loc, o.d_chunk);
+            t = q * (7 * o.chunk) + xcd * o.chunk + loc;
+        } else {
+            const int l2 = lin - o.full;
+            if (l2 < 8 * o.run) t = o.full + xcd * o.run + (l2 >> 3);
+        }
+    }
+    const int ip = (int)fdiv((uint32_t)t, o.d_tiles), tile = t - ip * o.tiles;
+    *item = (int)fdiv((uint32_t)ip, o.d_split);
+    *part = ip - *item * o.split;
+    const int g = (int)fdiv((uint32_t)tile, o.d_span), w = tile - g * (int)o.d_span.d;
+    const int left = o.tiles_m - g * o.group_m;
+    const bool whole = left >= o.group_m;
+    const int rows = whole ? o.group_m : left;
+    *tn = (int)fdiv((uint32_t)w, whole ? o.d_rows : o.d_last);
+    *tm = g * o.group_m + (w - *tn * rows);
+    *s0 = *part * o.steps + (*part < o.extra ? *part : o.extra);
+    *s1 = *s0 + o.steps + (*part < o.extra ? 1 : 0);
 }
 
 // Where each region lives inside the caller's workspace, and how the work is split. A batch
@@ -147,7 +195,7 @@ struct Layout {
     int band_groups;    // column groups of the band kernel (Np = band_groups * band_w)
     int split;          // split-K parts
     int xcd_chunk;      // contraction block order (xcd_order): blocks resident per XCD, or 0
-    int group_m;        // tile rows per group of the block order (block_tile)
+    int group_m;        // tile rows per group of the block order (block_of)
     bool ta, tb;
     bool a_strided, b_strided;  // operand read along k with a stride (column access)
     int nch_a, kch_a;   // row-max pass of op(A): chunks along K and chunk length

@@ -62,7 +62,7 @@ __device__ __forceinline__ float round_levels_exact(const int (&lv)[L], int E) {
 // fewer each: at S = 3 the first four levels reach K * 16129 (2^21 + 2 * 2^14 + 3 * 2^7 + 2)
 // = K * 3.4360e10, below 2^45 = 3.5184e13 for K <= 1023; at S = 2, K * 16129 (2^7 + 2), for K below
 // 2^24 (the int32 level sums end earlier); at S = 1 there is no such step.
-__host__ __device__ inline bool horner_exact(int S, int K) { return S < 3 || K <= 1023; }
+__host__ __device__ constexpr bool horner_exact(int S, int K) { return S < 3 || K <= 1023; }
 
 template <int L>
 __device__ __forceinline__ float round_levels(const int (&lv)[L], int E) {
