@@ -87,6 +87,10 @@ _SIGNATURES = {
                                        ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                        ctypes.POINTER(rg_config), ctypes.c_void_p, ctypes.c_size_t,
                                        ctypes.c_void_p, ctypes.c_void_p]),
+    "rg_gemm_bias_fp32_ws": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                            ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
+                                            ctypes.c_int, ctypes.POINTER(rg_config),
+                                            ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
     "rg_gemm_fp32_noalloc": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                             ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                             ctypes.POINTER(rg_config), ctypes.c_void_p]),
@@ -133,15 +137,27 @@ _SIGNATURES = {
     "rg_sum_fp32_ws": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                       ctypes.c_int, ctypes.c_int, ctypes.POINTER(rg_sum_config),
                                       ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "rg_sum_watch_fp32_ws": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
+                                            ctypes.c_int, ctypes.c_int,
+                                            ctypes.POINTER(rg_sum_config), ctypes.c_void_p,
+                                            ctypes.c_size_t, ctypes.c_void_p, ctypes.c_int,
+                                            ctypes.c_void_p]),
     "rg_sum_fp32": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                                    ctypes.c_int, ctypes.POINTER(rg_sum_config), ctypes.c_void_p]),
     "rg_scan_finite": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
                                       ctypes.c_int, ctypes.c_void_p]),
+    "rg_scan_finite_pair": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int,
+                                           ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int,
+                                           ctypes.c_void_p, ctypes.c_void_p]),
     "rg_conv_shape_init": (None, [ctypes.POINTER(rg_conv_shape)]),
     "rg_conv2d_workspace": _CONV_WS,
     "rg_conv2d_grad_weight_workspace": _CONV_WS,
     "rg_conv2d_grad_input_workspace": _CONV_WS,
     "rg_conv2d_ws": _CONV_RUN,
+    "rg_conv2d_bias_ws": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+                                         ctypes.c_void_p, ctypes.POINTER(rg_conv_shape),
+                                         ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t,
+                                         ctypes.c_void_p]),
     "rg_conv2d_grad_weight_ws": _CONV_RUN,
     "rg_conv2d_grad_input_ws": _CONV_RUN,
     "rg_test_conv_fused": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape), ctypes.c_int,

@@ -526,7 +526,7 @@ int gemm_launch(const float* A, const float* B, float* C, const Layout& L, char*
                         L.kch_b, pmb, qb, eb);
     da.nanrows = opt.nanrows_a;
     db.nanrows = opt.nanrows_b;
-    const OutAddr out{addr.ldc, addr.stride_c};
+    const OutAddr out{addr.ldc, addr.stride_c, addr.bias};
 
     if (L.band_w > 0) {  // op(B)'s one pass, then op(A)'s slicing, contraction, rounding
         if (opt.group_a > 0 || opt.group_b > 0 || opt.raw || opt.im2col_a || opt.nanrows_a ||
@@ -536,7 +536,7 @@ int gemm_launch(const float* A, const float* B, float* C, const Layout& L, char*
         launch_onepass(db, false, db, true, L.S, stream);
         record(1);
         launch_contract_band(L, A, addr.lda, static_cast<const int8_t*>(qb), eb, C, addr.ldc,
-                             stream);
+                             addr.bias, stream);
         record(2);
         record(3);
         return hipGetLastError();
@@ -828,6 +828,19 @@ int rg_gemm_fp32_ws(const float* A, const float* B, float* C, int M, int N, int 
                            rg::dense_addressing(L));
 }
 
+int rg_gemm_bias_fp32_ws(const float* A, const float* B, const float* bias, float* C, int M, int N, int K,
+                         const rg_config* cfg, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!A || !B || !C || !bias) return hipErrorInvalidValue;
+    rg::Layout L;
+    int e = rg::layout_for_current_device(M, N, K, cfg, &L);
+    if (e != hipSuccess) return e;
+    if (!workspace || workspace_bytes < L.total) return hipErrorInvalidValue;
+    rg::GemmAddressing addr = rg::dense_addressing(L);
+    addr.bias = bias;
+    return rg::gemm_launch(A, B, C, L, static_cast<char*>(workspace), static_cast<hipStream_t>(stream),
+                           nullptr, rg::GemmOptions(), addr);
+}
+
 int rg_gemm_fp32_noalloc(const float* A, const float* B, float* C, int M, int N, int K,
                          const rg_config* cfg, void* stream) {
     if (!A || !B || !C) return hipErrorInvalidValue;
@@ -871,7 +884,7 @@ int rg_gemm_strided_batched_fp32_ws(const float* A, long long lda, long long str
     if (lda < (L.ta ? M : K) || ldb < (L.tb ? K : N) || ldc < N) return hipErrorInvalidValue;
     if (stride_a < 0 || stride_b < 0 || stride_c < 0) return hipErrorInvalidValue;
     if (!workspace || workspace_bytes < L.total) return hipErrorInvalidValue;
-    rg::GemmAddressing addr{lda, ldb, ldc, stride_a, stride_b, stride_c};
+    rg::GemmAddressing addr{lda, ldb, ldc, stride_a, stride_b, stride_c, nullptr};
     return rg::gemm_launch(A, B, C, L, static_cast<char*>(workspace),
                            static_cast<hipStream_t>(stream), nullptr, rg::GemmOptions(), addr);
 }

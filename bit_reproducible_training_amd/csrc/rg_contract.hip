@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, (contract_waves_per_simd<S, WT
 contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
               const int* __restrict__ eA, const int* __restrict__ eB, float* __restrict__ C,
               int64_t* __restrict__ partial, int M, int N, int Kp, int Mp, int Np, long long ldc,
-              long long c_item, BlockOrder order) {
+              long long c_item, BlockOrder order, const float* __restrict__ bias) {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer resources exist only in the device pass
     constexpr int L = 2 * S - 1;
     constexpr int NW = WGM * WGN;                  // wavefronts per block
@@ -108,8 +108,16 @@ contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
     // row's exponent from its lane with a shuffle) and the exponents of its own columns. The
     // arrays cover the padded rows and columns, so the loads need no bounds check.
     const int e0 = -14 * (S - 1);
+    // bias (may be null): added to the rounded outputs of its column, one IEEE addition each; without
+    // one, -0.0 is added, which changes no value.
     int er_lane = 0;
     int ec[WTJ];
+    float bv[WTJ];
+#pragma unroll
+    for (int tj = 0; tj < WTJ; ++tj) {
+        const int c = tn * BN + (wn * WTJ + tj) * 32 + (lane & 31);
+        bv[tj] = bias != nullptr && c < N ? bias[c] : -0.0f;
+    }
     if (partial == nullptr) {
         er_lane = eA[tm * BM + wm * WTI * 32 + lane % (WTI * 32)];
 #pragma unroll
@@ -319,6 +327,8 @@ contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
                             v[i] = round_to_float_rare(combine_levels<L>(lv), er[4 * q + i] + ec[tj]);
                         }
                     }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] += bv[tj];
                     // Non-temporal stores: C is not read again here, and streaming it past the
                     // caches made the contraction faster (4096^3 steady state 0.466 -> 0.459 ms,
                     // 8192x3072x768 NT 0.166 -> 0.158 ms, LM-head forward -1.5%; A/B on one box).
@@ -393,7 +403,8 @@ struct SmallLds {
 template <int S>
 __global__ void __launch_bounds__(SMALL_THREADS, 1)
 contract_small(SmallOperand a, SmallOperand b, float* __restrict__ C, int K, long long ldc,
-               long long stride_a, long long stride_b, long long stride_c, int tiles_n) {
+               long long stride_a, long long stride_b, long long stride_c, int tiles_n,
+               const float* __restrict__ bias) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int L = 2 * S - 1;
     __shared__ v4i buf[SmallLds<S>::V4];
@@ -536,7 +547,8 @@ contract_small(SmallOperand a, SmallOperand b, float* __restrict__ C, int K, lon
             for (int w = 0; w < 4; ++w) v += red[((w * L + l) * 16 + e) * 64 + ln];
             lv[l] = v;
         }
-        C[(size_t)gr * ldc + gc] = round_levels<L>(lv, sexp[0][row] + sexp[1][col] + e0);
+        const float bv = bias != nullptr ? bias[gc] : -0.0f;  // (adding -0.0 changes no value)
+        C[(size_t)gr * ldc + gc] = round_levels<L>(lv, sexp[0][row] + sexp[1][col] + e0) + bv;
     }
 #endif
 }
@@ -560,7 +572,7 @@ template <int S, int NSL>
 __global__ void __launch_bounds__(BAND_THREADS, BAND_THREADS / 256)
 contract_band(const float* __restrict__ A, long long lda, int vec_a, const int8_t* __restrict__ QB,
               int qb_bytes, const int* __restrict__ eB, float* __restrict__ C, long long ldc,
-              int M, int N, int K, int Kp_ws, int W, int groups) {
+              int M, int N, int K, int Kp_ws, int W, int groups, const float* __restrict__ bias) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int L = 2 * S - 1;
     constexpr int D = BAND_DEPTH;
@@ -601,8 +613,14 @@ contract_band(const float* __restrict__ A, long long lda, int vec_a, const int8_
 #pragma unroll
     for (int d = 0; d < D; ++d)
         if (d < total) fetch(bq[d]);
-    int ec = 0;  // column exponent (lane % 32) of the current tile
-    if (total > 0) ec = eB[tile_of(0) * 32 + (lane & 31)];
+    int ec = 0;  // column exponent (lane % 32) and bias (-0.0, which changes no value, without one)
+    float bv = -0.0f;  // of the current tile
+    auto load_column = [&](int j) RG_INLINE {
+        const int c = tile_of(j) * 32 + (lane & 31);
+        ec = eB[c];
+        if (bias != nullptr) bv = bias[min(c, N - 1)];
+    };
+    if (total > 0) load_column(0);
 
     // Slicing of the band: slot i = t + BAND_THREADS j is lane s = i % 64 of k panel i / 64,
     // i.e. row s % 32 and k = 32 (i / 64) + 16 (s / 32) .. + 15. Every load is issued first.
@@ -707,6 +725,8 @@ contract_band(const float* __restrict__ A, long long lda, int vec_a, const int8_
                     v[i] = round_to_float_rare(combine_levels<L>(lv), er[4 * q + i] + ec);
                 }
             }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] += bv;
             if (col < N) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -736,7 +756,7 @@ contract_band(const float* __restrict__ A, long long lda, int vec_a, const int8_
             epilogue();
             ks = 0;
             ++jt;
-            if (jt < my_tiles) ec = eB[tile_of(jt) * 32 + (lane & 31)];
+            if (jt < my_tiles) load_column(jt);
         }
     };
     for (int it = 0; it < total; it += D) {
@@ -776,7 +796,8 @@ template <int TPO, int RU>
 __global__ void __launch_bounds__(256)
 reduce_round(const int64_t* __restrict__ partial, const int* __restrict__ eA,
              const int* __restrict__ eB, float* __restrict__ C, int M, int N, int split, int e0,
-             int batch, int Mp, int Np, long long ldc, long long c_item) {
+             int batch, int Mp, int Np, long long ldc, long long c_item,
+             const float* __restrict__ bias) {
     constexpr int OPB = 256 / TPO;  // outputs per block
     const int t = threadIdx.x;
     const int ol = t % OPB, sub = t / OPB;
@@ -784,6 +805,7 @@ reduce_round(const int64_t* __restrict__ partial, const int* __restrict__ eA,
     const size_t MN = (size_t)M * N;
     const bool live = idx < MN * batch;
     int item = 0, r = 0, c = 0, ea = 0, eb = 0;
+    float bv = -0.0f;  // (adding -0.0 changes no value)
     size_t rc = 0;
     int64_t acc = 0;
     if (live) {
@@ -794,6 +816,7 @@ reduce_round(const int64_t* __restrict__ partial, const int* __restrict__ eA,
             c = (int)(rc % N);
             ea = eA[(size_t)item * Mp + r];
             eb = eB[(size_t)item * Np + c];
+            if (bias != nullptr) bv = bias[c];
         }
         const int64_t* p0 = partial + (size_t)item * split * MN + rc;
         for (int p = sub; p < split; p += TPO * RU) {
@@ -816,7 +839,7 @@ reduce_round(const int64_t* __restrict__ partial, const int* __restrict__ eA,
         acc = red[t];  // complete for sub == 0, which wrote it last
     }
     if (live && sub == 0)
-        C[(size_t)item * c_item + (size_t)r * ldc + c] = round_output(acc, ea + eb + e0);
+        C[(size_t)item * c_item + (size_t)r * ldc + c] = round_output(acc, ea + eb + e0) + bv;
 }
 
 // Test hooks: the epilogue roundings on arrays. levels: n x (2S-1) int32, most significant
@@ -860,7 +883,7 @@ static void launch_mfma_s(const Layout& L, const int8_t* qa, const int8_t* qb, c
     // Block tiles: 128x128 = 8 wavefronts of 64x32; 128x64 and 64x128 = 8 wavefronts of 32x32
     // (two per SIMD); 64x64 = 4 wavefronts of 32x32; 64x192 and 192x64 = 12 wavefronts of
     // 32x32 (three per SIMD).
-#define RG_CONTRACT_ARGS qa, qb, ea, eb, C, partial, L.M, L.N, L.Kp, L.Mp, L.Np, out.ldc, out.c_item, order
+#define RG_CONTRACT_ARGS qa, qb, ea, eb, C, partial, L.M, L.N, L.Kp, L.Mp, L.Np, out.ldc, out.c_item, order, out.bias
     // (The twelve-wavefront tiles exist for S = 3 only: their 48 stage panels split evenly over
     // 12 wavefronts; the planner never gives them to S < 3.)
     if constexpr (S == 3) {
@@ -910,7 +933,7 @@ void launch_contract_small(const Layout& L, const float* A, const float* B, floa
     const dim3 grid((unsigned)(tiles_m * tiles_n), 1, (unsigned)L.batch);
 #define RG_SMALL(SS)                                                                            \
     contract_small<SS><<<grid, SMALL_THREADS, 0, stream>>>(a, b, C, L.K, addr.ldc, addr.stride_a, \
-                                                 addr.stride_b, addr.stride_c, tiles_n)
+                                                 addr.stride_b, addr.stride_c, tiles_n, addr.bias)
     switch (L.S) {
         case 1: RG_SMALL(1); break;
         case 2: RG_SMALL(2); break;
@@ -921,7 +944,7 @@ void launch_contract_small(const Layout& L, const float* A, const float* B, floa
 }
 
 void launch_contract_band(const Layout& L, const float* A, long long lda, const int8_t* qb,
-                          const int* eb, float* C, long long ldc, hipStream_t stream) {
+                          const int* eb, float* C, long long ldc, const float* bias, hipStream_t stream) {
     // 16-byte loads for rows that start 16-byte aligned with K % 4 == 0
     const int vec_a = (reinterpret_cast<uintptr_t>(A) & 15) == 0 && lda % 4 == 0 && L.K % 4 == 0;
     const int nkp = (L.K + PANEL_K - 1) / PANEL_K;
@@ -931,7 +954,7 @@ void launch_contract_band(const Layout& L, const float* A, long long lda, const 
 #define RG_BAND(SS, NS)                                                                         \
     contract_band<SS, NS><<<blocks, BAND_THREADS, 0, stream>>>(A, lda, vec_a, qb, qb_bytes, eb,  \
                                                               C, ldc, L.M, L.N, L.K, L.Kp,      \
-                                                              L.band_w, L.band_groups)
+                                                              L.band_w, L.band_groups, bias)
 #define RG_BAND_S(SS)                       \
     switch (nsl) {                          \
         case 1: RG_BAND(SS, 1); break;      \
@@ -974,10 +997,10 @@ void launch_reduce_round(const Layout& L, const int64_t* partial, const int* ea,
 #define RG_REDUCE(T)                                                                              \
     (many ? reduce_round<T, 8><<<blocks, 256, 0, stream>>>(partial, ea, eb, C, L.M, L.N, L.split,  \
                                                            -14 * (L.S - 1), L.batch, L.Mp, L.Np, \
-                                                           out.ldc, out.c_item)                 \
+                                                           out.ldc, out.c_item, out.bias)       \
           : reduce_round<T, 1><<<blocks, 256, 0, stream>>>(partial, ea, eb, C, L.M, L.N, L.split,  \
                                                            -14 * (L.S - 1), L.batch, L.Mp, L.Np, \
-                                                           out.ldc, out.c_item))
+                                                           out.ldc, out.c_item, out.bias))
     switch (tpo) {
         case 1: RG_REDUCE(1); break;
         case 4: RG_REDUCE(4); break;

@@ -166,10 +166,10 @@ __global__ void __launch_bounds__(THREADS) zero_flags_kernel(unsigned* __restric
 
 // dst[b][c][r] = src[b][r][c] for `batch` matrices of rows x cols, through a 32 x 33 LDS tile
 // so both the reads and the writes of a wavefront are consecutive. Grid: x over the 32 x 32
-// tiles of one matrix, y over the matrices.
+// tiles of one matrix, y over the matrices. bias[c] (or null) is added to the values of column c.
 __global__ void __launch_bounds__(THREADS)
 transpose_kernel(const float* __restrict__ src, float* __restrict__ dst, int rows, int cols,
-                 int tiles_c) {
+                 int tiles_c, const float* __restrict__ bias) {
     __shared__ float tile[32][33];
     const int tr = blockIdx.x / tiles_c, tc = blockIdx.x - tr * tiles_c;
     const size_t off = (size_t)blockIdx.y * rows * cols;
@@ -183,7 +183,10 @@ transpose_kernel(const float* __restrict__ src, float* __restrict__ dst, int row
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int c = tc * 32 + ty + 8 * i, r = tr * 32 + tx;
-        if (r < rows && c < cols) dst[off + (size_t)c * rows + r] = tile[tx][ty + 8 * i];
+        if (r < rows && c < cols) {
+            const float v = tile[tx][ty + 8 * i];
+            dst[off + (size_t)c * rows + r] = bias != nullptr ? v + bias[c] : v;
+        }
     }
 }
 
@@ -201,13 +204,15 @@ nfp_to_rows_kernel(const float* __restrict__ t, float* __restrict__ rows, Geom g
 
 // t[n][f][p] = rows[n * P + p][f] (GEMM output to NCHW).
 __global__ void __launch_bounds__(THREADS)
-rows_to_nfp_kernel(const float* __restrict__ rows, float* __restrict__ t, Geom g) {
+rows_to_nfp_kernel(const float* __restrict__ rows, float* __restrict__ t, Geom g,
+                   const float* __restrict__ bias) {
     const uint32_t total = (uint32_t)(g.windows * g.F);
     for (uint32_t i = blockIdx.x * THREADS + threadIdx.x; i < total; i += gridDim.x * THREADS) {
         const uint32_t n = fdiv(i, g.dFP);
         const uint32_t r = i - n * (uint32_t)(g.F * g.P);
         const uint32_t f = fdiv(r, g.dP), p = r - f * (uint32_t)g.P;
-        t[i] = rows[(n * (uint32_t)g.P + p) * (uint32_t)g.F + f];
+        const float v = rows[(n * (uint32_t)g.P + p) * (uint32_t)g.F + f];
+        t[i] = bias != nullptr ? v + bias[f] : v;
     }
 }
 
@@ -369,7 +374,7 @@ __device__ __forceinline__ void gather4(T* __restrict__ dst, const float* __rest
 template <int FC>
 __global__ void __launch_bounds__(THREADS)
 fwd_direct_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ out,
-                  Geom g, int S, FastDiv dtiles, int G, int Fp) {
+                  Geom g, int S, FastDiv dtiles, int G, int Fp, const float* __restrict__ bias) {
     extern __shared__ double wq[];                               // [K][Fp]
     int* ef = reinterpret_cast<int*>(wq + g.K * Fp);             // [F]
     const int nw = THREADS / G;
@@ -459,9 +464,10 @@ fwd_direct_kernel(const float* __restrict__ x, const float* __restrict__ w, floa
         const int nf = min(FC, g.F - f0);
 #pragma unroll
         for (int j = 0; j < FC; ++j)
-            if (j < nf)
-                out[((size_t)n * g.F + f0 + j) * g.P + p] =
-                    repro_gemm::round_to_float_f64((int64_t)acc[j], e0 + ef[f0 + j]);
+            if (j < nf) {
+                const float v = repro_gemm::round_to_float_f64((int64_t)acc[j], e0 + ef[f0 + j]);
+                out[((size_t)n * g.F + f0 + j) * g.P + p] = bias != nullptr ? v + bias[f0 + j] : v;
+            }
     }
 }
 
@@ -818,12 +824,13 @@ void launch_im2col(const float* x, float* cols, const Geom& g, unsigned* nanw, u
 
 // [N][F][P] -> [N * P][F] (to_rows) or back, as N transposes of F x P matrices; the element-
 // wise kernels when N exceeds the grid's y range.
-void launch_nfp_rows(const float* src, float* dst, const Geom& g, bool to_rows, hipStream_t stream) {
+void launch_nfp_rows(const float* src, float* dst, const Geom& g, bool to_rows, const float* bias,
+                     hipStream_t stream) {
     const int rows = to_rows ? g.F : g.P, cols = to_rows ? g.P : g.F;
     if (g.N <= 65535) {
         const int tiles_r = (rows + 31) / 32, tiles_c = (cols + 31) / 32;
         hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)(tiles_r * tiles_c), (unsigned)g.N),
-                           dim3(THREADS), 0, stream, src, dst, rows, cols, tiles_c);
+                           dim3(THREADS), 0, stream, src, dst, rows, cols, tiles_c, bias);
         return;
     }
     const size_t outn = (size_t)g.windows * g.F;
@@ -832,11 +839,13 @@ void launch_nfp_rows(const float* src, float* dst, const Geom& g, bool to_rows, 
                            stream, src, dst, g);
     else
         hipLaunchKernelGGL(rows_to_nfp_kernel, dim3((unsigned)grid_for(outn)), dim3(THREADS), 0,
-                           stream, src, dst, g);
+                           stream, src, dst, g, bias);
 }
 
+// bias: one float per filter added to the forward pass's rounded outputs, or null.
 int run_pass(Kind kind, const float* a, const float* b, float* out, const rg_conv_shape* s, int S,
-             int algo, void* workspace, size_t workspace_bytes, void* stream_) {
+             int algo, void* workspace, size_t workspace_bytes, void* stream_,
+             const float* bias = nullptr) {
     if (!a || !b || !out) return hipErrorInvalidValue;
     ConvPlan p;
     int e = conv_plan(kind, s, S, algo, &p);
@@ -852,10 +861,10 @@ int run_pass(Kind kind, const float* a, const float* b, float* out, const rg_con
             const int G = fwd_groups(g.F), Fp = fwd_padded_filters(g.F);
             const size_t lds = fwd_lds_bytes(g);
             switch (fwd_pass_width(g.F)) {
-                case 1: fwd_direct_kernel<1><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp); break;
-                case 2: fwd_direct_kernel<2><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp); break;
-                case 4: fwd_direct_kernel<4><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp); break;
-                default: fwd_direct_kernel<8><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp); break;
+                case 1: fwd_direct_kernel<1><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp, bias); break;
+                case 2: fwd_direct_kernel<2><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp, bias); break;
+                case 4: fwd_direct_kernel<4><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp, bias); break;
+                default: fwd_direct_kernel<8><<<grid, THREADS, lds, stream>>>(a, b, out, g, S, dt, G, Fp, bias); break;
             }
         } else {
             const long long tiles = dx_tiles_per_plane(g);
@@ -869,7 +878,7 @@ int run_pass(Kind kind, const float* a, const float* b, float* out, const rg_con
         return hipGetLastError();
     }
     char* base = static_cast<char*>(workspace);
-    if (p.fused) return fused_launch(p.f, a, b, out, base, stream);
+    if (p.fused) return fused_launch(p.f, a, b, bias, out, base, stream);
     if (p.dwfused) return dw_launch(p.d, a, b, out, base, stream);
     char* gws = base + p.gemm;
     switch (kind) {
@@ -896,13 +905,13 @@ int run_pass(Kind kind, const float* a, const float* b, float* out, const rg_con
                                 dense_addressing(p.L));
             }
             if (e != hipSuccess) return e;
-            launch_nfp_rows(yrows, out, g, false, stream);
+            launch_nfp_rows(yrows, out, g, false, bias, stream);
             break;
         }
         case Kind::GradWeight: {
             float* dyrows = reinterpret_cast<float*>(base + p.buf0);
             float* cols = reinterpret_cast<float*>(base + p.buf1);
-            launch_nfp_rows(a, dyrows, g, true, stream);
+            launch_nfp_rows(a, dyrows, g, true, nullptr, stream);
             // Positions holding a NaN in some window take exponent 0 (raw-bit maxima).
             GemmOptions opt;
             unsigned* nank = zero_flags(p, base, stream);
@@ -915,7 +924,7 @@ int run_pass(Kind kind, const float* a, const float* b, float* out, const rg_con
         }
         case Kind::GradInput: {
             float* dyrows = reinterpret_cast<float*>(base + p.buf0);
-            launch_nfp_rows(a, dyrows, g, true, stream);
+            launch_nfp_rows(a, dyrows, g, true, nullptr, stream);
             GemmOptions opt;
             opt.group_a = g.K;   // rows of op(A) are the positions: one scale for all weights
             opt.group_b = g.P;   // rows of op(B)^T are the windows: one scale per image
@@ -977,6 +986,14 @@ int rg_conv2d_ws(const float* x, const float* weight, float* out, const rg_conv_
                  void* workspace, size_t workspace_bytes, void* stream) {
     return rg::run_pass(rg::Kind::Forward, x, weight, out, s, S, RG_CONV_ALGO_AUTO, workspace,
                         workspace_bytes, stream);
+}
+
+int rg_conv2d_bias_ws(const float* x, const float* weight, const float* bias, float* out,
+                      const rg_conv_shape* s, int S, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+    if (!bias) return hipErrorInvalidValue;
+    return rg::run_pass(rg::Kind::Forward, x, weight, out, s, S, RG_CONV_ALGO_AUTO, workspace,
+                        workspace_bytes, stream, bias);
 }
 
 int rg_conv2d_grad_weight_ws(const float* dy, const float* x, float* dw, const rg_conv_shape* s,

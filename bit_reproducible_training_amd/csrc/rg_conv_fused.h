@@ -64,8 +64,9 @@ struct FusedPlan {
 // RG_CONV_GRAD_INPUT; the shape is valid).
 bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, FusedPlan* plan);
 
-// a: x (forward) or dY; w: the layer's weights; out: y or dX.
-int fused_launch(const FusedPlan& p, const float* a, const float* w, float* out, char* ws,
-                 hipStream_t stream);
+// a: x (forward) or dY; w: the layer's weights; bias: one float per output channel, added to the
+// rounded outputs, or null; out: y or dX.
+int fused_launch(const FusedPlan& p, const float* a, const float* w, const float* bias, float* out,
+                 char* ws, hipStream_t stream);
 
 }  // namespace rg

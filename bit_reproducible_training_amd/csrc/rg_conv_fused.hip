@@ -262,11 +262,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t output_rsrc(const FusedPlan& p
 // holds channel 8 (e / 4) + 4 (lane / 32) + e % 4, position lane % 32. sef: the tiles' channel
 // exponents (less 14 (S - 1)); f0: the first channel; er: the lane's position's exponent; o: its
 // output at channel 0 (bytes from the block's first image, whose resource is orsrc; an offset past
-// its range for a position that is not stored). exact: horner_exact, uniform.
+// its range for a position that is not stored). exact: horner_exact, uniform. sbias: the tiles'
+// channel biases, added to the rounded outputs, or null.
 template <int S, int TF>
 __device__ __forceinline__ void store_tiles(const v16i (&acc)[2 * S - 1][TF], const int* sef, int f0, int F,
                                             uint32_t plane4, int er, __amdgpu_buffer_rsrc_t orsrc,
-                                            uint32_t o, bool exact, bool partial) {
+                                            uint32_t o, bool exact, bool partial, const float* sbias) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int L = 2 * S - 1;
     const int lane = threadIdx.x & 63;
@@ -327,6 +328,10 @@ __device__ __forceinline__ void store_tiles(const v16i (&acc)[2 * S - 1][TF], co
                     }
                 }
             }
+            if (sbias != nullptr) {  // uniform
+#pragma unroll
+                for (int i = 0; i < 4; ++i) val[i] += sbias[fl + 8 * q + i];
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t so = (uint32_t)(f0 + ti * 32 + 8 * q + i) * plane4;
@@ -353,7 +358,7 @@ __device__ __forceinline__ void store_tiles(const v16i (&acc)[2 * S - 1][TF], co
 template <int S, int TF, int NWW, int NWF, bool FORWARD>
 __global__ void __launch_bounds__(64 * NWW * NWF, 2)
 fused_contract(FusedPlan p, const float* __restrict__ src, const char* __restrict__ ws,
-               float* __restrict__ out) {
+               float* __restrict__ out, const float* __restrict__ bias) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int L = 2 * S - 1;
     constexpr int NW = NWW * NWF;
@@ -369,10 +374,11 @@ fused_contract(FusedPlan p, const float* __restrict__ src, const char* __restric
     // took have the fast rounding.
     constexpr int BF = 32 * TF * NWF;              // output channels per block
     __shared__ v4i lds[2 * (PP + PQ) + 2][64];
-    static_assert(BW + BF + NW <= 512, "exponents and flags fit two panels");
+    static_assert(BW + 2 * BF + NW <= 512, "exponents, flags and biases fit two panels");
     int* sexp = reinterpret_cast<int*>(lds[2 * (PP + PQ)]);
     int* sef = sexp + BW;
     int* sfast = sef + BF;
+    float* sbias = reinterpret_cast<float*>(sfast + NW);
 
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -508,7 +514,10 @@ fused_contract(FusedPlan p, const float* __restrict__ src, const char* __restric
         const bool any_slow = __ballot(slow) != 0;
         if (lane == 0) sfast[wave] = !any_slow;
         const int* ef = reinterpret_cast<const int*>(ws + p.ef) + ft * BF;
-        if (t < BF) sef[t] = ef[t] - 14 * (S - 1);
+        if (t < BF) {
+            sef[t] = ef[t] - 14 * (S - 1);
+            if (bias != nullptr) sbias[t] = ft * BF + t < p.F ? bias[ft * BF + t] : 0.0f;
+        }
     }
     __syncthreads();
     int allfast = 1;  // the SUB wavefronts that took this group's exponents
@@ -608,7 +617,8 @@ fused_contract(FusedPlan p, const float* __restrict__ src, const char* __restric
     if (FORWARD && p.split > 1 && part == 0 && ft == 0 && wf == 0 && lane < 32 && r < c.rows)
         reinterpret_cast<int*>(const_cast<char*>(ws) + p.ew)[(size_t)n * p.OPL + gy * p.OW + gx] = sexp[ww * 32 + lane];
     store_tiles<S, TF>(acc, sef + wf * TF * 32, ft * BF + wf * TF * 32, p.F, oplane4,
-                       sexp[ww * 32 + (lane & 31)], output_rsrc(p, out, ws, part, n0), o, p.exact != 0, p.split > 1);
+                       sexp[ww * 32 + (lane & 31)], output_rsrc(p, out, ws, part, n0), o, p.exact != 0, p.split > 1,
+                       bias != nullptr ? sbias + wf * TF * 32 : nullptr);
 #endif
 }
 
@@ -628,7 +638,7 @@ fused_contract(FusedPlan p, const float* __restrict__ src, const char* __restric
 template <int S, int TF, bool FORWARD>
 __global__ void __launch_bounds__(256, 2)
 fused_patch(FusedPlan p, const float* __restrict__ src, const char* __restrict__ ws,
-            float* __restrict__ out) {
+            float* __restrict__ out, const float* __restrict__ bias) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int L = 2 * S - 1;
     constexpr int NW = 4, BW = 32 * NW, BF = 32 * TF;
@@ -638,12 +648,13 @@ fused_patch(FusedPlan p, const float* __restrict__ src, const char* __restrict__
     // outstanding copies): patches, channel panels, positions' exponents, channels' exponents and
     // the positions' slow flags.
     constexpr int PATCH4 = 16 * PX / 4;            // v4i per patch slot
-    __shared__ v4i lds[2 * PATCH4 + 2 * PQ * 64 + (2 * BW + BF) / 4];
+    __shared__ v4i lds[2 * PATCH4 + 2 * PQ * 64 + (2 * BW + 2 * BF) / 4];
     float* patch = reinterpret_cast<float*>(lds);
     v4i* panels = lds + 2 * PATCH4;
     int* sexp = reinterpret_cast<int*>(panels + 2 * PQ * 64);
     int* sslow = sexp + BW;
     int* sef = sslow + BW;
+    float* sbias = reinterpret_cast<float*>(sef + BF);
 
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -739,6 +750,7 @@ fused_patch(FusedPlan p, const float* __restrict__ src, const char* __restrict__
         const int n = (int)fdiv((uint32_t)img, c.dNS), strip = img - n * c.NS;
         uint32_t key = 0, raw = 0;
         const int ef = t < BF ? reinterpret_cast<const int*>(ws + p.ef)[ft * BF + t] : 0;
+        const float bv = bias != nullptr && t < BF && ft * BF + t < p.F ? bias[ft * BF + t] : 0.0f;
         auto first_copies = [&]() RG_INLINE {
             __builtin_amdgcn_sched_barrier(0);
             copy_panels(s0);
@@ -780,7 +792,10 @@ fused_patch(FusedPlan p, const float* __restrict__ src, const char* __restrict__
             sexp[pos] = se;
             sslow[pos] = !(raw < 0x7F800000u && n2 >= -126 && n2 <= 127);
         }
-        if (t < BF) sef[t] = ef - 14 * (S - 1);
+        if (t < BF) {
+            sef[t] = ef - 14 * (S - 1);
+            if (bias != nullptr) sbias[t] = bv;
+        }
     }
 
     v16i acc[L][TF];
@@ -901,14 +916,15 @@ fused_patch(FusedPlan p, const float* __restrict__ src, const char* __restrict__
     if (FORWARD && p.split > 1 && part == 0 && ft == 0 && lane < 32 && o != NOWHERE)
         reinterpret_cast<int*>(const_cast<char*>(ws) + p.ew)[(size_t)n * p.OPL + gy * p.OW + gx] = se;
     store_tiles<S, TF>(acc, sef, ft * BF, p.F, oplane4, se, output_rsrc(p, out, ws, part, n0), o, p.exact != 0,
-                       p.split > 1);
+                       p.split > 1, bias != nullptr ? sbias : nullptr);
 #endif
 }
 
 // Adds the parts' exact sums and rounds once: out[n][f][pixel] (FusedPlan::split > 1).
 template <bool FORWARD>
 __global__ void __launch_bounds__(THREADS)
-fused_reduce(FusedPlan p, const char* __restrict__ ws, float* __restrict__ out) {
+fused_reduce(FusedPlan p, const char* __restrict__ ws, float* __restrict__ out,
+             const float* __restrict__ bias) {
     const uint32_t total = (uint32_t)p.N * p.F * p.OPL;
     const uint32_t i = blockIdx.x * THREADS + threadIdx.x;
     if (i >= total) return;
@@ -925,7 +941,8 @@ fused_reduce(FusedPlan p, const char* __restrict__ ws, float* __restrict__ out) 
     const int ep = FORWARD ? reinterpret_cast<const int*>(ws + p.ew)[n * (uint32_t)p.OPL + pix]
                            : repro_gemm::scale_exponent(
                                  __uint_as_float(reinterpret_cast<const uint2*>(ws + p.imax)[n].x));
-    out[i] = round_output(sum, ep + reinterpret_cast<const int*>(ws + p.ef)[f] - 14 * (p.S - 1));
+    const float v = round_output(sum, ep + reinterpret_cast<const int*>(ws + p.ef)[f] - 14 * (p.S - 1));
+    out[i] = bias != nullptr ? v + bias[f] : v;
 }
 
 }  // namespace
@@ -1118,8 +1135,8 @@ bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, FusedPlan*
 }
 
 template <int S>
-static void launch_s(const FusedPlan& p, const float* a, const float* w, float* out, char* ws,
-                     hipStream_t stream) {
+static void launch_s(const FusedPlan& p, const float* a, const float* w, const float* bias, float* out,
+                     char* ws, hipStream_t stream) {
     if (p.input_grad) {
         fused_dx_maxima<<<(unsigned)p.maxima_blocks, THREADS, 0, stream>>>(p, a, w, ws);
         fused_dx_weights<S><<<(unsigned)(p.qblocks + ceil_div(p.N, THREADS / 64)), THREADS, 0, stream>>>(p, w, ws);
@@ -1128,16 +1145,16 @@ static void launch_s(const FusedPlan& p, const float* a, const float* w, float* 
     }
     if (p.patch) {
 #define RG_PATCH(TF)                                                                             \
-    (p.input_grad ? fused_patch<S, TF, false><<<(unsigned)(p.blocks * p.split), 256, 0, stream>>>(p, a, ws, out) \
-                  : fused_patch<S, TF, true><<<(unsigned)(p.blocks * p.split), 256, 0, stream>>>(p, a, ws, out))
+    (p.input_grad ? fused_patch<S, TF, false><<<(unsigned)(p.blocks * p.split), 256, 0, stream>>>(p, a, ws, out, bias) \
+                  : fused_patch<S, TF, true><<<(unsigned)(p.blocks * p.split), 256, 0, stream>>>(p, a, ws, out, bias))
         if (p.tf == 2) RG_PATCH(2);
         else RG_PATCH(1);
 #undef RG_PATCH
     } else {
 #define RG_FUSED(TF, NWF)                                                                        \
     (p.input_grad                                                                                \
-         ? fused_contract<S, TF, 4, NWF, false><<<(unsigned)(p.blocks * p.split), 256 * NWF, 0, stream>>>(p, a, ws, out) \
-         : fused_contract<S, TF, 4, NWF, true><<<(unsigned)(p.blocks * p.split), 256 * NWF, 0, stream>>>(p, a, ws, out))
+         ? fused_contract<S, TF, 4, NWF, false><<<(unsigned)(p.blocks * p.split), 256 * NWF, 0, stream>>>(p, a, ws, out, bias) \
+         : fused_contract<S, TF, 4, NWF, true><<<(unsigned)(p.blocks * p.split), 256 * NWF, 0, stream>>>(p, a, ws, out, bias))
     if (p.nwf == 2) RG_FUSED(2, 2);
     else if (p.tf == 2) RG_FUSED(2, 1);
     else RG_FUSED(1, 1);
@@ -1145,17 +1162,17 @@ static void launch_s(const FusedPlan& p, const float* a, const float* w, float* 
     }
     if (p.split > 1) {
         const unsigned blocks = (unsigned)ceil_div((long long)p.N * p.F * p.OPL, THREADS);
-        if (p.input_grad) fused_reduce<false><<<blocks, THREADS, 0, stream>>>(p, ws, out);
-        else fused_reduce<true><<<blocks, THREADS, 0, stream>>>(p, ws, out);
+        if (p.input_grad) fused_reduce<false><<<blocks, THREADS, 0, stream>>>(p, ws, out, bias);
+        else fused_reduce<true><<<blocks, THREADS, 0, stream>>>(p, ws, out, bias);
     }
 }
 
-int fused_launch(const FusedPlan& p, const float* a, const float* w, float* out, char* ws,
-                 hipStream_t stream) {
+int fused_launch(const FusedPlan& p, const float* a, const float* w, const float* bias, float* out,
+                 char* ws, hipStream_t stream) {
     switch (p.S) {
-        case 1: launch_s<1>(p, a, w, out, ws, stream); break;
-        case 2: launch_s<2>(p, a, w, out, ws, stream); break;
-        case 3: launch_s<3>(p, a, w, out, ws, stream); break;
+        case 1: launch_s<1>(p, a, w, bias, out, ws, stream); break;
+        case 2: launch_s<2>(p, a, w, bias, out, ws, stream); break;
+        case 3: launch_s<3>(p, a, w, bias, out, ws, stream); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -398,6 +398,7 @@ int layout_for_current_device(int M, int N, int K, const rg_config* cfg, Layout*
 struct GemmAddressing {
     long long lda, ldb, ldc;
     long long stride_a, stride_b, stride_c;
+    const float* bias = nullptr;  // see OutAddr (a single GEMM's)
 };
 GemmAddressing dense_addressing(const Layout& L);
 
@@ -419,6 +420,7 @@ void launch_group_max2(const SliceDesc* a, int group_a, const SliceDesc* b, int 
 // C + b * c_item, rows ldc apart.
 struct OutAddr {
     long long ldc, c_item;
+    const float* bias = nullptr;  // N values added to the rounded outputs of their columns, or null
 };
 void launch_contract_mfma(const Layout& L, const int8_t* qa, const int8_t* qb, const int* ea,
                           const int* eb, float* C, OutAddr out, int64_t* partial,
@@ -429,7 +431,7 @@ void launch_contract_small(const Layout& L, const float* A, const float* B, floa
 // Slicing of op(A), contraction and rounding in one launch, for a layout with L.band_w > 0
 // (op(B)'s digit panels qb and exponents eb already in the workspace).
 void launch_contract_band(const Layout& L, const float* A, long long lda, const int8_t* qb,
-                          const int* eb, float* C, long long ldc, hipStream_t stream);
+                          const int* eb, float* C, long long ldc, const float* bias, hipStream_t stream);
 void launch_contract_reference(const Layout& L, const int32_t* xa, const int32_t* xb,
                                int64_t* partial, hipStream_t stream);
 void launch_reduce_round(const Layout& L, const int64_t* partial, const int* ea, const int* eb,

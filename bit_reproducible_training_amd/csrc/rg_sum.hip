@@ -202,10 +202,25 @@ struct ThreadSum {
 
 // C == 1. Block = 64 outputs (lanes) x 4 row phases (waves); chunk = blockIdx.y covers rows
 // [a0, a1), phase w takes rows a0 + w, a0 + w + 4, ...
+// Lowers flag[0] to op_id if any of the wave's lanes holds `bad`: one atomic per such wave.
+__device__ inline void report(bool bad, int* flag, int op_id) {
+    const unsigned long long votes = __ballot(bad);
+    if (votes != 0 && (threadIdx.x & 63) == (unsigned)(__ffsll((long long)votes) - 1))
+        atomicMin(flag, op_id);
+}
+
+// watch (in this kernel and the next): the pass that reads the values also reports a NaN or an
+// infinity among them, as scan_nonfinite does (watch.flag null: no report). A bias gradient and the
+// check of the incoming gradient are then one read of it: 8192 x 3072, 17 us of scan saved.
+struct Watch {
+    int* flag;
+    int op_id;
+};
+
 __global__ void __launch_bounds__(SUM_THREADS)
 sum_columns(const float* __restrict__ x, int A, int B, int rows_per_chunk, int chunks,
             uint32_t divisor, float* __restrict__ out, int64_t* __restrict__ part,
-            int* __restrict__ part_nf) {
+            int* __restrict__ part_nf, Watch watch) {
     __shared__ int64_t acc[LIMBS * SUM_THREADS];
     __shared__ int nf_sh[SUM_THREADS];
     const int t = threadIdx.x, col = t & 63, phase = t >> 6;
@@ -226,6 +241,7 @@ sum_columns(const float* __restrict__ x, int A, int B, int rows_per_chunk, int c
         }
     }
     sum.finish();
+    if (watch.flag != nullptr) report(sum.nonfinite != 0, watch.flag, watch.op_id);
     nf_sh[t] = sum.nonfinite;
     __syncthreads();
     // The four phases' limbs: thread t adds limb (t >> 6) + 4 i of output t & 63.
@@ -256,7 +272,8 @@ sum_columns(const float* __restrict__ x, int A, int B, int rows_per_chunk, int c
 template <bool VEC>
 __global__ void __launch_bounds__(SUM_THREADS)
 sum_segments(const float* __restrict__ x, int A, int B, int C, FastDiv dC, int chunks, uint32_t divisor,
-             float* __restrict__ out, int64_t* __restrict__ part, int* __restrict__ part_nf) {
+             float* __restrict__ out, int64_t* __restrict__ part, int* __restrict__ part_nf,
+             Watch watch) {
     __shared__ int64_t acc[LIMBS * SUM_THREADS];
     __shared__ int64_t merged[4][LIMBS];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -313,11 +330,13 @@ sum_segments(const float* __restrict__ x, int A, int B, int C, FastDiv dC, int c
             // A zero sum is +0.0; a NaN among the values gives the NaN of repro_sum::finalize.
             const bool nan = !(__builtin_fabs(s) < __builtin_inf());
             out[b] = nan ? __uint_as_float(0x7FC00000u) : (s == 0.0 ? 0.0f : (float)s);
+            if (nan && watch.flag != nullptr) atomicMin(watch.flag, watch.op_id);
         }
         return;
     }
     sum.finish();
     const int nf = __ballot(sum.nonfinite != 0) != 0;
+    if (nf && lane == 0 && watch.flag != nullptr) atomicMin(watch.flag, watch.op_id);
     // Limb l of the wave: four lanes add 16 threads' limbs each. (A wave's LDS operations are in
     // order, and only this wave's threads' limbs are read.)
     __builtin_amdgcn_wave_barrier();
@@ -429,13 +448,27 @@ __device__ inline bool is_nonfinite(float v) {
     return (repro_gemm::float_to_bits(v) & 0x7F800000u) == 0x7F800000u;
 }
 
+// The n floats at x, op_id the number reported for them, by `blocks` blocks of a scan.
+struct ScanPart {
+    const float* x;
+    size_t n;
+    int vec;
+    int op_id;
+    unsigned blocks;
+};
+
+// Two arrays' scans in one launch (the second may be empty, with no blocks): a layer checks its
+// input and its weight with one launch instead of two.
 __global__ void __launch_bounds__(SUM_THREADS)
-scan_nonfinite(const float* __restrict__ x, size_t n, int vec, int* flag, int op_id) {
-    const size_t tid = (size_t)blockIdx.x * SUM_THREADS + threadIdx.x;
-    const size_t stride = (size_t)gridDim.x * SUM_THREADS;
+scan_nonfinite(ScanPart p0, ScanPart p1, int* flag) {
+    const bool second = blockIdx.x >= p0.blocks;
+    const float* __restrict__ x = second ? p1.x : p0.x;
+    const size_t n = second ? p1.n : p0.n;
+    const size_t tid = (size_t)(blockIdx.x - (second ? p0.blocks : 0)) * SUM_THREADS + threadIdx.x;
+    const size_t stride = (size_t)(second ? p1.blocks : p0.blocks) * SUM_THREADS;
     bool bad = false;
     size_t tail = 0;
-    if (vec) {
+    if (second ? p1.vec : p0.vec) {
         const size_t n4 = n / 4;
         const float4* x4 = reinterpret_cast<const float4*>(x);
         for (size_t i = tid; i < n4; i += stride) {
@@ -446,9 +479,14 @@ scan_nonfinite(const float* __restrict__ x, size_t n, int vec, int* flag, int op
         tail = 4 * n4;
     }
     for (size_t i = tail + tid; i < n; i += stride) bad = bad || is_nonfinite(x[i]);
-    const unsigned long long votes = __ballot(bad);
-    if (votes != 0 && (threadIdx.x & 63) == (unsigned)(__ffsll((long long)votes) - 1))
-        atomicMin(flag, op_id);
+    report(bad, flag, second ? p1.op_id : p0.op_id);
+}
+
+ScanPart scan_part(const float* x, size_t n, int op_id) {
+    ScanPart p{x, n, (reinterpret_cast<uintptr_t>(x) & 15) == 0, op_id, 0};
+    const size_t per_block = (size_t)SUM_THREADS * (p.vec ? 16 : 4);
+    p.blocks = (unsigned)std::min<size_t>((n + per_block - 1) / per_block, 4096);
+    return p;
 }
 
 struct SumLayout {
@@ -534,7 +572,13 @@ int rg_sum_plan_for_device(int A, int B, int C, const rg_sum_config* cfg, int nu
 }
 
 int rg_sum_fp32_ws(const float* x, float* out, int A, int B, int C, const rg_sum_config* cfg,
-                   void* workspace, size_t workspace_bytes, void* stream_) {
+                   void* workspace, size_t workspace_bytes, void* stream) {
+    return rg_sum_watch_fp32_ws(x, out, A, B, C, cfg, workspace, workspace_bytes, nullptr, 0, stream);
+}
+
+int rg_sum_watch_fp32_ws(const float* x, float* out, int A, int B, int C, const rg_sum_config* cfg,
+                         void* workspace, size_t workspace_bytes, int* flag, int op_id,
+                         void* stream_) {
     if (!x || !out) return hipErrorInvalidValue;
     rg::SumLayout L;
     const int e = rg::sum_layout_current(A, B, C, cfg, &L);
@@ -542,20 +586,22 @@ int rg_sum_fp32_ws(const float* x, float* out, int A, int B, int C, const rg_sum
     if (L.total && (!workspace || workspace_bytes < L.total)) return hipErrorInvalidValue;
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     const uint32_t divisor = cfg->mean ? (uint32_t)((long long)A * C) : 1u;
+    const rg::Watch watch{flag, op_id};
     int64_t* part = L.total ? static_cast<int64_t*>(workspace) : nullptr;
     int* part_nf = L.total ? reinterpret_cast<int*>(static_cast<char*>(workspace) + L.nf_offset)
                            : nullptr;
     if (L.columns) {
         dim3 grid((B + 63) / 64, L.chunks);
         hipLaunchKernelGGL(rg::sum_columns, grid, dim3(rg::SUM_THREADS), 0, stream, x, A, B,
-                           L.rows_per_chunk, L.chunks, divisor, out, part, part_nf);
+                           L.rows_per_chunk, L.chunks, divisor, out, part, part_nf, watch);
     } else {
         const long long items = (long long)B * L.chunks;
         if ((items + 3) / 4 > INT_MAX) return hipErrorInvalidValue;
         const bool vec = C % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
         const auto segments = vec ? rg::sum_segments<true> : rg::sum_segments<false>;
         hipLaunchKernelGGL(segments, dim3((unsigned)((items + 3) / 4)), dim3(rg::SUM_THREADS), 0, stream,
-                           x, A, B, C, rg::make_fastdiv((uint32_t)C), L.chunks, divisor, out, part, part_nf);
+                           x, A, B, C, rg::make_fastdiv((uint32_t)C), L.chunks, divisor, out, part, part_nf,
+                           watch);
     }
     if (L.chunks > 1) {
         if (L.chunks < rg::MERGE_BLOCK_FROM)
@@ -581,14 +627,17 @@ int rg_sum_fp32(const float* x, float* out, int A, int B, int C, const rg_sum_co
     return e;
 }
 
-int rg_scan_finite(const float* x, int* flag, size_t n, int op_id, void* stream_) {
-    if (n == 0) return hipSuccess;
-    if (!x || !flag) return hipErrorInvalidValue;
-    const int vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-    const size_t per_block = (size_t)rg::SUM_THREADS * (vec ? 16 : 4);
-    const size_t blocks = std::min<size_t>((n + per_block - 1) / per_block, 4096);
-    hipLaunchKernelGGL(rg::scan_nonfinite, dim3((unsigned)blocks), dim3(rg::SUM_THREADS), 0,
-                       static_cast<hipStream_t>(stream_), x, n, vec, flag, op_id);
+int rg_scan_finite(const float* x, int* flag, size_t n, int op_id, void* stream) {
+    return rg_scan_finite_pair(x, n, op_id, nullptr, 0, 0, flag, stream);
+}
+
+int rg_scan_finite_pair(const float* x, size_t nx, int op_x, const float* y, size_t ny, int op_y,
+                        int* flag, void* stream_) {
+    if (nx == 0 && ny == 0) return hipSuccess;
+    if ((nx && !x) || (ny && !y) || !flag) return hipErrorInvalidValue;
+    const rg::ScanPart p0 = rg::scan_part(x, nx, op_x), p1 = rg::scan_part(y, ny, op_y);
+    hipLaunchKernelGGL(rg::scan_nonfinite, dim3(p0.blocks + p1.blocks), dim3(rg::SUM_THREADS), 0,
+                       static_cast<hipStream_t>(stream_), p0, p1, flag);
     return hipGetLastError();
 }
 

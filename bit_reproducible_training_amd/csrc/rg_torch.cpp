@@ -63,11 +63,24 @@ Tensor workspace_like(size_t bytes, const Tensor& t) {
     return torch::empty({(int64_t)std::max<size_t>(bytes, 1)}, t.options().dtype(torch::kUInt8));
 }
 
+// A layer's bias (or none) that a library call can add in its own launches: n contiguous floats on
+// the operands' device. Any other (a broadcastable shape, another type or stride) is added by a
+// PyTorch operation.
+const float* fusible_bias(const c10::optional<Tensor>& bias, const Tensor& a, int64_t n) {
+    if (!bias.has_value()) return nullptr;
+    const Tensor& b = *bias;
+    const bool ok = b.scalar_type() == torch::kFloat32 && b.device() == a.device() && b.dim() == 1 &&
+                    b.size(0) == n && b.is_contiguous();
+    return ok ? b.data_ptr<float>() : nullptr;
+}
+
 // C[M, N] = op(A) op(B) (bindings.cpp:43-66), with the planner's options exposed: split_k,
 // the block tile and the algorithm change the speed, never a bit; they apply to GPU tensors.
 // out, when given, must be a contiguous float32 tensor of M*N elements on A's device.
-Tensor gemm_ex(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S, int split_k,
-               int tile_m, int tile_n, int algo, c10::optional<Tensor> out) {
+// bias, when given, is added to the rows of C, one rounding per output (an out is not given then).
+Tensor gemm_run(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S, int split_k,
+                int tile_m, int tile_n, int algo, c10::optional<Tensor> out,
+                c10::optional<Tensor> bias) {
     require_f32(A, "A");
     require_f32(B, "B");
     const bool gpu = on_gpu(A, B, "gemm");
@@ -98,10 +111,16 @@ Tensor gemm_ex(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S,
         rg_plan plan;
         check(rg_make_plan(M, N, K, &cfg, &plan), "gemm plan");
         Tensor ws = workspace_like(plan.workspace_bytes, A);
+        if (const float* b = fusible_bias(bias, A, N)) {
+            check(rg_gemm_bias_fp32_ws(A.data_ptr<float>(), B.data_ptr<float>(), b, C.data_ptr<float>(),
+                                       M, N, K, &cfg, ws.data_ptr(), (size_t)ws.numel(), stream_of(A)),
+                  "gemm");
+            return C;
+        }
         check(rg_gemm_fp32_ws(A.data_ptr<float>(), B.data_ptr<float>(), C.data_ptr<float>(), M, N, K,
                               &cfg, ws.data_ptr(), (size_t)ws.numel(), stream_of(A), nullptr),
               "gemm");
-        return C;
+        return bias.has_value() ? C + *bias : C;
     }
     need(S >= 1 && S <= 3, "gemm: slices must be 1..3");
     const float* a = A.data_ptr<float>();
@@ -109,7 +128,17 @@ Tensor gemm_ex(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S,
     float* c = C.data_ptr<float>();
     py::gil_scoped_release nogil;
     repro_gemm::cpu_gemm(a, b, c, M, N, K, ta, tb, S);
-    return C;
+    return bias.has_value() ? C + *bias : C;
+}
+
+Tensor gemm_ex(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S, int split_k,
+               int tile_m, int tile_n, int algo, c10::optional<Tensor> out) {
+    return gemm_run(A, B, M, N, K, ta, tb, S, split_k, tile_m, tile_n, algo, out, c10::nullopt);
+}
+
+// y[M, N] = x[M, K] w[N, K]^T, plus bias (or None).
+Tensor linear(Tensor x, Tensor w, c10::optional<Tensor> bias, int M, int N, int K, int S) {
+    return gemm_run(x, w, M, N, K, false, true, S, 1, 16, 16, RG_ALGO_AUTO, c10::nullopt, bias);
 }
 
 Tensor gemm(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S) {
@@ -118,7 +147,8 @@ Tensor gemm(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S) {
 
 // out[b] = exact sum over a, c of x[a, b, c], rounded once; divided by A * C if mean
 // (bindings.cpp:69-91).
-Tensor exact_sum(Tensor x, int A, int B, int C, bool mean) {
+// flag, when given, is also lowered to op_id if x holds a NaN or infinity (GPU tensors only).
+Tensor sum_run(Tensor x, int A, int B, int C, bool mean, c10::optional<Tensor> flag, int op_id) {
     require_f32(x, "x");
     need(x.is_cuda() || x.is_cpu(), "sum: x must be on the CPU or a GPU");
     x = x.contiguous();
@@ -133,8 +163,10 @@ Tensor exact_sum(Tensor x, int A, int B, int C, bool mean) {
         rg_sum_plan plan;
         check(rg_make_sum_plan(A, B, C, &cfg, &plan), "sum plan");
         Tensor ws = workspace_like(plan.workspace_bytes, x);
-        check(rg_sum_fp32_ws(x.data_ptr<float>(), out.data_ptr<float>(), A, B, C, &cfg, ws.data_ptr(),
-                             (size_t)ws.numel(), stream_of(x)),
+        check(rg_sum_watch_fp32_ws(x.data_ptr<float>(), out.data_ptr<float>(), A, B, C, &cfg,
+                                   ws.data_ptr(), (size_t)ws.numel(),
+                                   flag.has_value() ? flag->data_ptr<int>() : nullptr, op_id,
+                                   stream_of(x)),
               "sum");
         return out;
     }
@@ -143,6 +175,23 @@ Tensor exact_sum(Tensor x, int A, int B, int C, bool mean) {
     py::gil_scoped_release nogil;
     repro_sum::cpu_sum(p, o, A, B, C, mean);
     return out;
+}
+
+Tensor exact_sum(Tensor x, int A, int B, int C, bool mean) {
+    return sum_run(x, A, B, C, mean, c10::nullopt, 0);
+}
+
+void require_flag(const Tensor& flag, const Tensor& x, const char* op) {
+    need(flag.scalar_type() == torch::kInt32 && flag.numel() >= 1,
+         std::string(op) + ": flag must be an int32 tensor");
+    need(on_gpu(x, flag, op), std::string(op) + ": tensors must be on a GPU");
+}
+
+// exact_sum and scan_finite of one GPU tensor in one read of it.
+Tensor exact_sum_watch(Tensor x, int A, int B, int C, Tensor flag, int op_id) {
+    require_f32(x, "x");
+    require_flag(flag, x, "exact_sum_watch");
+    return sum_run(x, A, B, C, false, flag, op_id);
 }
 
 repro_conv::ConvShape shape_of(const std::vector<int64_t>& x_shape, int F, int KH, int KW, int SY,
@@ -164,10 +213,10 @@ repro_conv::ConvShape shape_of(const std::vector<int64_t>& x_shape, int F, int K
 }
 
 typedef int (*ConvWorkspaceFn)(const rg_conv_shape*, int, size_t*);
-typedef int (*ConvRunFn)(const float*, const float*, float*, const rg_conv_shape*, int, void*, size_t, void*);
 
 // One convolution pass on the GPU: plan, per-call workspace, launch on the current stream.
-void conv_gpu(ConvWorkspaceFn ws_fn, ConvRunFn run, const Tensor& a, const Tensor& b, Tensor& out,
+template <class Run>
+void conv_gpu(ConvWorkspaceFn ws_fn, Run run, const Tensor& a, const Tensor& b, Tensor& out,
               const repro_conv::ConvShape& g, int S, const char* what) {
     c10::DeviceGuard guard(a.device());
     const rg_conv_shape s = g.to_c();
@@ -180,7 +229,9 @@ void conv_gpu(ConvWorkspaceFn ws_fn, ConvRunFn run, const Tensor& a, const Tenso
 }
 
 // out[N][F][OH][OW] from x[N][C][H][W] and w[F][C][KH][KW] (bindings.cpp:112-131).
-Tensor conv2d(Tensor x, Tensor w, int SY, int SX, int PY, int PX, int S) {
+// bias, when given, is added to the channels of out, one rounding per output.
+Tensor conv2d_bias(Tensor x, Tensor w, c10::optional<Tensor> bias, int SY, int SX, int PY, int PX,
+                   int S) {
     require_f32(x, "x");
     require_f32(w, "weight");
     const bool gpu = on_gpu(x, w, "conv2d");
@@ -192,14 +243,27 @@ Tensor conv2d(Tensor x, Tensor w, int SY, int SX, int PY, int PX, int S) {
     need(repro_conv::cpu_shape_valid(g, S), "conv2d: invalid shape");
     Tensor out = torch::empty({g.N, g.F, g.OH(), g.OW()}, x.options());
     if (gpu) {
+        const float* b = fusible_bias(bias, x, g.F);
+        const auto fused = [b](const float* px, const float* pw, float* po, const rg_conv_shape* s,
+                               int S, void* ws, size_t bytes, void* stream) {
+            return rg_conv2d_bias_ws(px, pw, b, po, s, S, ws, bytes, stream);
+        };
+        if (b != nullptr) {
+            conv_gpu(rg_conv2d_workspace, fused, x, w, out, g, S, "conv");
+            return out;
+        }
         conv_gpu(rg_conv2d_workspace, rg_conv2d_ws, x, w, out, g, S, "conv");
-        return out;
+        return bias.has_value() ? out + bias->view({1, -1, 1, 1}) : out;
     }
     const float *px = x.data_ptr<float>(), *pw = w.data_ptr<float>();
     float* po = out.data_ptr<float>();
     py::gil_scoped_release nogil;
     repro_conv::cpu_conv2d(px, pw, po, g, S);
-    return out;
+    return bias.has_value() ? out + bias->view({1, -1, 1, 1}) : out;
+}
+
+Tensor conv2d(Tensor x, Tensor w, int SY, int SX, int PY, int PX, int S) {
+    return conv2d_bias(x, w, c10::nullopt, SY, SX, PY, PX, S);
 }
 
 // dW[F][C][KH][KW] from dY[N][F][OH][OW] and x (bindings.cpp:133-152).
@@ -276,6 +340,20 @@ void scan_finite(Tensor x, Tensor flag, int op_id) {
     }
 }
 
+// scan_finite of two GPU tensors in one launch.
+void scan_finite_pair(Tensor x, int op_x, Tensor y, int op_y, Tensor flag) {
+    require_f32(x, "x");
+    require_f32(y, "x");
+    require_flag(flag, x, "scan_finite");
+    require_flag(flag, y, "scan_finite");
+    x = x.contiguous();
+    y = y.contiguous();
+    c10::DeviceGuard guard(x.device());
+    check(rg_scan_finite_pair(x.data_ptr<float>(), (size_t)x.numel(), op_x, y.data_ptr<float>(),
+                              (size_t)y.numel(), op_y, flag.data_ptr<int>(), stream_of(x)),
+          "finite scan");
+}
+
 }  // namespace
 
 // 64-bit FNV-1a over the raw bytes of a contiguous CPU tensor, continuing from h: the hash the
@@ -302,6 +380,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("conv2d_grad_weight", &conv2d_grad_weight);
     m.def("conv2d_grad_input", &conv2d_grad_input);
     m.def("scan_finite", &scan_finite);
+    // The layers' forms: the same operations with fewer launches.
+    m.def("linear", &linear);
+    m.def("conv2d_bias", &conv2d_bias);
+    m.def("exact_sum_watch", &exact_sum_watch);
+    m.def("scan_finite_pair", &scan_finite_pair);
     m.def("cpu_threads", &repro_gemm::cpu_thread_count);
     m.def("set_error_class", [](py::object cls) {
         Py_XINCREF(cls.ptr());

@@ -19,7 +19,9 @@ Design:
     inside one step.
   - Inputs and weights are checked for NaN/Inf by the module before the autograd function
     runs, incoming gradients inside backward; the checks are queued kernels (GPU) or a loop
-    (CPU) that never synchronise.
+    (CPU) that never synchronise. On a GPU input and weight share a launch, and a gradient
+    whose bias sum is wanted is checked by that sum's read of it.
+  - On a GPU the bias is added in the launch that rounds the outputs.
   - Linear accepts any number of leading dimensions ([..., in_features]), flattened into the
     GEMM's rows.
 """
@@ -27,7 +29,8 @@ from dataclasses import dataclass
 
 import torch
 
-from .repro_conv import conv2d, conv2d_grad_input, conv2d_grad_weight
+from ._lib import _backend
+from .repro_conv import conv2d_grad_input, conv2d_grad_weight
 from .repro_gemm import gemm
 from .repro_sum import exact_sum, scan_finite
 
@@ -79,6 +82,24 @@ class FiniteGuard:
         """Queues a check of `tensor` under `label`."""
         scan_finite(tensor.detach(), self._cell(tensor.device), self._number(label))
 
+    def _scan_pair(self, x, label_x, y, label_y):
+        """scan(x, label_x) and scan(y, label_y); one launch where both are on one GPU."""
+        if not x.is_cuda or x.device != y.device:
+            self.scan(x, label_x)
+            self.scan(y, label_y)
+            return
+        number_x, number_y = self._number(label_x), self._number(label_y)
+        _backend.scan_finite_pair(x.detach(), number_x, y.detach(), number_y,
+                                  self._cell(x.device))
+
+    def _scan_and_sum(self, dy, label, a, b, c):
+        """scan(dy, label), and the exact sum of the contiguous dy as [a][b][c] over a and c; one
+        read of dy on a GPU."""
+        if not dy.is_cuda:
+            self.scan(dy, label)
+            return exact_sum(dy, a, b, c, False)
+        return _backend.exact_sum_watch(dy, a, b, c, self._cell(dy.device), self._number(label))
+
     def first_offender(self):
         """The first label (in order of first use) that met a NaN or infinity, or None."""
         worst = min((int(c.item()) for c in self._cells.values()), default=self.CLEAN)
@@ -126,8 +147,7 @@ class _CallInfo:
 
 
 def _watch_operands(info, x, weight):
-    info.guard.scan(x, info.name + " input")
-    info.guard.scan(weight, info.name + " weight")
+    info.guard._scan_pair(x, info.name + " input", weight, info.name + " weight")
 
 
 class _LinearOp(torch.autograd.Function):
@@ -136,8 +156,7 @@ class _LinearOp(torch.autograd.Function):
     @staticmethod
     def forward(x2d, weight, bias, info):
         m, k = x2d.shape
-        y = gemm(x2d, weight, m, weight.shape[0], k, False, True, info.slices)
-        return y if bias is None else y + bias
+        return _backend.linear(x2d, weight, bias, m, weight.shape[0], k, info.slices)
 
     @staticmethod
     def setup_context(ctx, inputs, output):
@@ -149,14 +168,17 @@ class _LinearOp(torch.autograd.Function):
     def backward(ctx, dy):
         x2d, weight = ctx.saved_tensors
         info = ctx.info
-        info.guard.scan(dy, info.name + " gradient")
         dy = dy.contiguous()
         m, k = x2d.shape
         n = weight.shape[0]
         want_x, want_w, want_b, _ = ctx.needs_input_grad
+        db = None
+        if want_b:
+            db = info.guard._scan_and_sum(dy, info.name + " gradient", m, n, 1)
+        else:
+            info.guard.scan(dy, info.name + " gradient")
         dx = gemm(dy, weight, m, k, n, False, False, info.slices) if want_x else None
         dw = gemm(dy, x2d, n, k, m, True, False, info.slices) if want_w else None
-        db = exact_sum(dy, m, n, 1, False) if want_b else None
         return dx, dw, db, None
 
 
@@ -179,8 +201,8 @@ class _ConvOp(torch.autograd.Function):
 
     @staticmethod
     def forward(x, weight, bias, stride, padding, info):
-        y = conv2d(x, weight, stride[0], stride[1], padding[0], padding[1], info.slices)
-        return y if bias is None else y + bias.view(1, -1, 1, 1)
+        return _backend.conv2d_bias(x, weight, bias, stride[0], stride[1], padding[0], padding[1],
+                                    info.slices)
 
     @staticmethod
     def setup_context(ctx, inputs, output):
@@ -194,18 +216,19 @@ class _ConvOp(torch.autograd.Function):
         x, weight = ctx.saved_tensors
         (sy, sx), (py, px) = ctx.geometry
         info = ctx.info
-        info.guard.scan(dy, info.name + " gradient")
         dy = dy.contiguous()
         want_x, want_w, want_b = ctx.needs_input_grad[:3]
         dx = dw = db = None
+        if want_b:
+            n, f, oh, ow = dy.shape
+            db = info.guard._scan_and_sum(dy, info.name + " gradient", n, f, oh * ow)
+        else:
+            info.guard.scan(dy, info.name + " gradient")
         if want_x:
             dx = conv2d_grad_input(dy, weight, list(x.shape), sy, sx, py, px, info.slices)
         if want_w:
             dw = conv2d_grad_weight(dy, x, weight.shape[2], weight.shape[3], sy, sx, py, px,
                                     info.slices)
-        if want_b:
-            n, f, oh, ow = dy.shape
-            db = exact_sum(dy, n, f, oh * ow, False)
         return dx, dw, db, None, None, None
 
 

@@ -60,6 +60,11 @@ int rg_conv2d_grad_input_workspace(const rg_conv_shape* g, int S, size_t* bytes)
  * position's maximum, which then takes exponent 0). */
 int rg_conv2d_ws(const float* x, const float* weight, float* out, const rg_conv_shape* g, int S,
                  void* workspace, size_t workspace_bytes, void* stream);
+/* rg_conv2d_ws followed by one IEEE addition per output, out[n][f][p] = fl(out[n][f][p] + bias[f]) for
+ * F floats of bias, in the convolution's own launches; the same workspace. 1 for a null bias. */
+int rg_conv2d_bias_ws(const float* x, const float* weight, const float* bias, float* out,
+                      const rg_conv_shape* g, int S, void* workspace, size_t workspace_bytes,
+                      void* stream);
 int rg_conv2d_grad_weight_ws(const float* dy, const float* x, float* dw, const rg_conv_shape* g,
                              int S, void* workspace, size_t workspace_bytes, void* stream);
 int rg_conv2d_grad_input_ws(const float* dy, const float* weight, float* dx,

@@ -84,6 +84,13 @@ int rg_gemm_fp32_ws(const float* A, const float* B, float* C, int M, int N, int 
                     const rg_config* cfg, void* workspace, size_t workspace_bytes, void* stream,
                     void* const* stage_events);
 
+/* rg_gemm_fp32_ws followed by one IEEE addition per output, C[r][c] = fl(C[r][c] + bias[c]) for N
+ * floats of bias (a Linear layer's forward pass), in the GEMM's own launches; the same plan and
+ * workspace. Errors as rg_gemm_fp32_ws, plus 1 for a null bias. No counterpart in the reference,
+ * whose layers add the bias with a PyTorch operation (the same bits). */
+int rg_gemm_bias_fp32_ws(const float* A, const float* B, const float* bias, float* C, int M, int N, int K,
+                         const rg_config* cfg, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Replaces repro_gemm::repro_gemm_fp32 (repro_gemm_cuda/repro_gemm.cuh:69-73,
  * repro_gemm.cu:530-542): allocates the workspace, runs, synchronises the stream to
  * surface asynchronous errors, frees. */

@@ -54,6 +54,11 @@ int rg_sum_plan_for_device(int A, int B, int C, const rg_sum_config* cfg, int nu
 int rg_sum_fp32_ws(const float* x, float* out, int A, int B, int C, const rg_sum_config* cfg,
                    void* workspace, size_t workspace_bytes, void* stream);
 
+/* rg_sum_fp32_ws that, in the same read of x, also does what rg_scan_finite(x, flag, A*B*C, op_id)
+ * does; a null flag reports nothing. */
+int rg_sum_watch_fp32_ws(const float* x, float* out, int A, int B, int C, const rg_sum_config* cfg,
+                         void* workspace, size_t workspace_bytes, int* flag, int op_id, void* stream);
+
 /* Replaces repro_sum::repro_sum_fp32 (repro_sum_cuda/repro_sum.cuh:43-45,
  * repro_sum.cu:261-271): allocates the workspace, runs, synchronises the stream, frees. */
 int rg_sum_fp32(const float* x, float* out, int A, int B, int C, const rg_sum_config* cfg,
@@ -63,6 +68,10 @@ int rg_sum_fp32(const float* x, float* out, int A, int B, int C, const rg_sum_co
  * *flag to op_id if x[0..n) holds a NaN or infinity; stream-ordered, never synchronises.
  * n == 0 launches nothing. 1 (invalid value): null x or flag with n > 0. */
 int rg_scan_finite(const float* x, int* flag, size_t n, int op_id, void* stream);
+
+/* rg_scan_finite of x under op_x and of y under op_y in one launch. */
+int rg_scan_finite_pair(const float* x, size_t nx, int op_x, const float* y, size_t ny, int op_y,
+                        int* flag, void* stream);
 
 #ifdef __cplusplus
 }
