@@ -551,7 +551,11 @@ __global__ void __launch_bounds__(256) split_kernel(SliceDesc a, SliceDesc b) {
 // stores). Wavefront w covers k in [32*NF4*w, 32*NF4*(w+1)) for all 8 rows; instruction i
 // covers its k-panel i:
 //   row access    lane L loads row L/8, k = 4*(L%8)..+3 of the panel: 8 rows x 128 bytes;
-//   column access lane L loads k = L/2 of the panel, columns 4*(L%2)..+3: 32 k-rows x 32 bytes.
+//   column access lane L loads k = L/2 of the panel, columns 4*(L%2)..+3: 32 k-rows x 32 bytes;
+//                 where the rows are not 16-byte aligned, four scalar loads of column L%8,
+//                 k = L/8 + 8*j: 8 k-rows x 32 bytes each, so a panel touches each of its cache
+//                 lines once (with the four scalars along a lane's columns every load touched 32
+//                 lines: 2049 x 1003 and 2049 x 3001, S = 2: AAAA).
 // The rows' maxima are reduced with lane shuffles and across the 8 wavefronts in LDS, then each
 // lane rounds 4 values and writes their digits as one 4-byte word per digit plane: for row
 // access the lane's own values (four consecutive lanes fill a 16-byte run, eight rows a
@@ -665,6 +669,25 @@ __device__ __forceinline__ void slice_onepass(const SliceDesc& d, long long blk)
         for (int off = 1; off < 8; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
         if (WS) wmax = m;  // lanes 8j..8j+7 all hold row j's maximum
         else if ((lane & 7) == 0) smax[w][lane >> 3] = m;
+    } else if (!d.vec) {  // column access, unaligned or R % 4 != 0
+        const int c = r0 + (lane & 7);
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NF4; ++i) {
+            float x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int k = (kp0 + i) * PANEL_K + 8 * j + (lane >> 3);
+                x[j] = k < d.K && c < d.R ? base[(size_t)k * d.ld + c] : 0.0f;
+            }
+            v[i] = make_float4(x[0], x[1], x[2], x[3]);
+        }
+#pragma unroll
+        for (int i = 0; i < NF4; ++i) m = fmaxf(m, max4(v[i]));
+#pragma unroll
+        for (int off = 8; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+        if (WS) wmax = __shfl(m, lane >> 3, 64);
+        else if (lane < 8) smax[w][lane] = m;
     } else {
         const int c = r0 + 4 * (lane & 1);
         float4 m = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -674,14 +697,7 @@ __device__ __forceinline__ void slice_onepass(const SliceDesc& d, long long blk)
             v[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (k < d.K && c < d.R) {
                 const float* q = base + (size_t)k * d.ld + c;
-                if (d.vec) {
-                    v[i] = *reinterpret_cast<const float4*>(q);
-                } else {  // unaligned or R % 4 != 0: four scalar loads inside R
-                    v[i].x = q[0];
-                    if (c + 1 < d.R) v[i].y = q[1];
-                    if (c + 2 < d.R) v[i].z = q[2];
-                    if (c + 3 < d.R) v[i].w = q[3];
-                }
+                v[i] = *reinterpret_cast<const float4*>(q);
             }
         }
 #pragma unroll
@@ -742,13 +758,18 @@ __device__ __forceinline__ void slice_onepass(const SliceDesc& d, long long blk)
         if (kp >= npk) break;
         float x[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
         if (d.strided) {
-            // this lane's k-row lane/2, columns 4*(lane%2)..+3 -> tile[column][k-row]; then
+            // this lane's values -> tile[column][k-row]; then
             // lane L takes column L/8, k = 4*(L%8)..+3
-            const int c4 = 4 * (lane & 1), kr = lane >> 1;
-            tile[c4 + 0][kr] = x[0];
-            tile[c4 + 1][kr] = x[1];
-            tile[c4 + 2][kr] = x[2];
-            tile[c4 + 3][kr] = x[3];
+            if (d.vec) {
+                const int c4 = 4 * (lane & 1), kr = lane >> 1;
+                tile[c4 + 0][kr] = x[0];
+                tile[c4 + 1][kr] = x[1];
+                tile[c4 + 2][kr] = x[2];
+                tile[c4 + 3][kr] = x[3];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) tile[lane & 7][8 * j + (lane >> 3)] = x[j];
+            }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
