@@ -37,7 +37,10 @@ constexpr int contract_waves_per_simd() {
     return w < need ? need : (w > cap ? cap : w);
 }
 
-template <int S, int WTI, int WTJ, int WGM, int WGN>
+// BIAS: bias[c] is added to the rounded outputs of column c, one IEEE addition each. (An instantiation
+// of its own: with the null pointer tested or -0.0 added instead, GEMMs without a bias took 0.3-0.9%
+// longer, 4096^3 435.5 -> 438.6 us.)
+template <int S, int WTI, int WTJ, int WGM, int WGN, bool BIAS>
 __global__ void __launch_bounds__(64 * WGM * WGN, (contract_waves_per_simd<S, WTI, WTJ, WGM, WGN>()))
 contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
               const int* __restrict__ eA, const int* __restrict__ eB, float* __restrict__ C,
@@ -108,15 +111,13 @@ contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
     // row's exponent from its lane with a shuffle) and the exponents of its own columns. The
     // arrays cover the padded rows and columns, so the loads need no bounds check.
     const int e0 = -14 * (S - 1);
-    // bias (may be null): added to the rounded outputs of its column, one IEEE addition each; without
-    // one, -0.0 is added, which changes no value.
     int er_lane = 0;
     int ec[WTJ];
     float bv[WTJ];
+    if constexpr (BIAS) {
 #pragma unroll
-    for (int tj = 0; tj < WTJ; ++tj) {
-        const int c = tn * BN + (wn * WTJ + tj) * 32 + (lane & 31);
-        bv[tj] = bias != nullptr && c < N ? bias[c] : -0.0f;
+        for (int tj = 0; tj < WTJ; ++tj)
+            bv[tj] = bias[min(tn * BN + (wn * WTJ + tj) * 32 + (lane & 31), N - 1)];
     }
     if (partial == nullptr) {
         er_lane = eA[tm * BM + wm * WTI * 32 + lane % (WTI * 32)];
@@ -327,8 +328,10 @@ contract_mfma(const int8_t* __restrict__ QA, const int8_t* __restrict__ QB,
                             v[i] = round_to_float_rare(combine_levels<L>(lv), er[4 * q + i] + ec[tj]);
                         }
                     }
+                    if constexpr (BIAS) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] += bv[tj];
+                        for (int i = 0; i < 4; ++i) v[i] += bv[tj];
+                    }
                     // Non-temporal stores: C is not read again here, and streaming it past the
                     // caches made the contraction faster (4096^3 steady state 0.466 -> 0.459 ms,
                     // 8192x3072x768 NT 0.166 -> 0.158 ms, LM-head forward -1.5%; A/B on one box).
@@ -400,7 +403,7 @@ struct SmallLds {
     static constexpr int V4 = (PANELS * 64 > RED * 16 ? PANELS * 64 : RED * 16);  // in v4i
 };
 
-template <int S>
+template <int S, bool BIAS>
 __global__ void __launch_bounds__(SMALL_THREADS, 1)
 contract_small(SmallOperand a, SmallOperand b, float* __restrict__ C, int K, long long ldc,
                long long stride_a, long long stride_b, long long stride_c, int tiles_n,
@@ -547,8 +550,9 @@ contract_small(SmallOperand a, SmallOperand b, float* __restrict__ C, int K, lon
             for (int w = 0; w < 4; ++w) v += red[((w * L + l) * 16 + e) * 64 + ln];
             lv[l] = v;
         }
-        const float bv = bias != nullptr ? bias[gc] : -0.0f;  // (adding -0.0 changes no value)
-        C[(size_t)gr * ldc + gc] = round_levels<L>(lv, sexp[0][row] + sexp[1][col] + e0) + bv;
+        float v = round_levels<L>(lv, sexp[0][row] + sexp[1][col] + e0);
+        if constexpr (BIAS) v += bias[gc];
+        C[(size_t)gr * ldc + gc] = v;
     }
 #endif
 }
@@ -872,7 +876,7 @@ void launch_test_round(const int* levels, const int64_t* T, const int* E, float*
     else round_levels_kernel<5><<<blocks, 256, 0, stream>>>(levels, E, out, n);
 }
 
-template <int S>
+template <int S, bool BIAS>
 static void launch_mfma_s(const Layout& L, const int8_t* qa, const int8_t* qb, const int* ea,
                           const int* eb, float* C, OutAddr out, int64_t* partial,
                           hipStream_t stream) {
@@ -888,34 +892,39 @@ static void launch_mfma_s(const Layout& L, const int8_t* qa, const int8_t* qb, c
     // 12 wavefronts; the planner never gives them to S < 3.)
     if constexpr (S == 3) {
         if (L.ti == 1 && L.tj == 3) {
-            contract_mfma<S, 1, 1, 2, 6><<<grid, 768, 0, stream>>>(RG_CONTRACT_ARGS);
+            contract_mfma<S, 1, 1, 2, 6, BIAS><<<grid, 768, 0, stream>>>(RG_CONTRACT_ARGS);
             return;
         }
         if (L.ti == 3 && L.tj == 1) {
-            contract_mfma<S, 1, 1, 6, 2><<<grid, 768, 0, stream>>>(RG_CONTRACT_ARGS);
+            contract_mfma<S, 1, 1, 6, 2, BIAS><<<grid, 768, 0, stream>>>(RG_CONTRACT_ARGS);
             return;
         }
     }
     if (L.ti == 2 && L.tj == 2)
-        contract_mfma<S, 2, 1, 2, 4><<<grid, 512, 0, stream>>>(RG_CONTRACT_ARGS);
+        contract_mfma<S, 2, 1, 2, 4, BIAS><<<grid, 512, 0, stream>>>(RG_CONTRACT_ARGS);
     else if (L.ti == 2 && L.tj == 1)
-        contract_mfma<S, 1, 1, 4, 2><<<grid, 512, 0, stream>>>(RG_CONTRACT_ARGS);
+        contract_mfma<S, 1, 1, 4, 2, BIAS><<<grid, 512, 0, stream>>>(RG_CONTRACT_ARGS);
     else if (L.ti == 1 && L.tj == 2)
-        contract_mfma<S, 1, 1, 2, 4><<<grid, 512, 0, stream>>>(RG_CONTRACT_ARGS);
+        contract_mfma<S, 1, 1, 2, 4, BIAS><<<grid, 512, 0, stream>>>(RG_CONTRACT_ARGS);
     else
-        contract_mfma<S, 1, 1, 2, 2><<<grid, 256, 0, stream>>>(RG_CONTRACT_ARGS);
+        contract_mfma<S, 1, 1, 2, 2, BIAS><<<grid, 256, 0, stream>>>(RG_CONTRACT_ARGS);
 #undef RG_CONTRACT_ARGS
 }
 
 void launch_contract_mfma(const Layout& L, const int8_t* qa, const int8_t* qb, const int* ea,
                           const int* eb, float* C, OutAddr out, int64_t* partial,
                           hipStream_t stream) {
+    const bool bias = out.bias != nullptr && partial == nullptr;  // (partials: the reduction adds it)
+#define RG_MFMA_S(SS)                                                                       \
+    (bias ? launch_mfma_s<SS, true>(L, qa, qb, ea, eb, C, out, partial, stream)             \
+          : launch_mfma_s<SS, false>(L, qa, qb, ea, eb, C, out, partial, stream))
     switch (L.S) {
-        case 1: launch_mfma_s<1>(L, qa, qb, ea, eb, C, out, partial, stream); break;
-        case 2: launch_mfma_s<2>(L, qa, qb, ea, eb, C, out, partial, stream); break;
-        case 3: launch_mfma_s<3>(L, qa, qb, ea, eb, C, out, partial, stream); break;
+        case 1: RG_MFMA_S(1); break;
+        case 2: RG_MFMA_S(2); break;
+        case 3: RG_MFMA_S(3); break;
         default: break;
     }
+#undef RG_MFMA_S
 }
 
 void launch_contract_small(const Layout& L, const float* A, const float* B, float* C,
@@ -932,8 +941,11 @@ void launch_contract_small(const Layout& L, const float* A, const float* B, floa
                          vec(B, addr.ldb, addr.stride_b, L.b_strided) ? 1 : 0};
     const dim3 grid((unsigned)(tiles_m * tiles_n), 1, (unsigned)L.batch);
 #define RG_SMALL(SS)                                                                            \
-    contract_small<SS><<<grid, SMALL_THREADS, 0, stream>>>(a, b, C, L.K, addr.ldc, addr.stride_a, \
-                                                 addr.stride_b, addr.stride_c, tiles_n, addr.bias)
+    (addr.bias != nullptr                                                                       \
+         ? contract_small<SS, true><<<grid, SMALL_THREADS, 0, stream>>>(                        \
+               a, b, C, L.K, addr.ldc, addr.stride_a, addr.stride_b, addr.stride_c, tiles_n, addr.bias) \
+         : contract_small<SS, false><<<grid, SMALL_THREADS, 0, stream>>>(                       \
+               a, b, C, L.K, addr.ldc, addr.stride_a, addr.stride_b, addr.stride_c, tiles_n, nullptr))
     switch (L.S) {
         case 1: RG_SMALL(1); break;
         case 2: RG_SMALL(2); break;
