@@ -17,6 +17,7 @@
 // partial (split-K, or a caller that wants the exact integers).
 // Integer addition is associative, so the tile shape, the split and the order of k
 // never change T.
+#include "rg_digits.h"
 #include "rg_internal.h"
 #include <type_traits>
 #include "repro_gemm_math.h"
@@ -485,23 +486,13 @@ contract_small(SmallOperand a, SmallOperand b, float* __restrict__ C, int K, lon
             const int rem = i - o * npk * 64;
             const int kp = rem >> 6, s = rem & 63;
             const RowScale rs = row_scale<S>(sexp[o][s & 31]);
-            int dg[S][16];
+            int X[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                int d[S];
-                digits_of<S>(round_fixed(x[j][e], rs), d);
+            for (int e = 0; e < 16; ++e) X[e] = round_fixed(x[j][e], rs);
+            v4i dg[S];
+            pack16<S>(X, dg);
 #pragma unroll
-                for (int p = 0; p < S; ++p) dg[p][e] = d[p];
-            }
-#pragma unroll
-            for (int p = 0; p < S; ++p) {
-                v4i w;
-                w[0] = (int)pack4(dg[p][0], dg[p][1], dg[p][2], dg[p][3]);
-                w[1] = (int)pack4(dg[p][4], dg[p][5], dg[p][6], dg[p][7]);
-                w[2] = (int)pack4(dg[p][8], dg[p][9], dg[p][10], dg[p][11]);
-                w[3] = (int)pack4(dg[p][12], dg[p][13], dg[p][14], dg[p][15]);
-                buf[((o * S + p) * npk + kp) * 64 + s] = w;
-            }
+            for (int p = 0; p < S; ++p) buf[((o * S + p) * npk + kp) * 64 + s] = dg[p];
         }
     }
     __syncthreads();
@@ -673,23 +664,13 @@ contract_band(const float* __restrict__ A, long long lda, int vec_a, const int8_
         const int kp = i >> 6, s = i & 63;
         if (kp < nkp) {
             const RowScale rs = row_scale<S>(sexp[s & 31]);
-            int dg[S][16];
+            int X[16];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                int dd[S];
-                digits_of<S>(round_fixed(x[j][e], rs), dd);
+            for (int e = 0; e < 16; ++e) X[e] = round_fixed(x[j][e], rs);
+            v4i dg[S];
+            pack16<S>(X, dg);
 #pragma unroll
-                for (int p = 0; p < S; ++p) dg[p][e] = dd[p];
-            }
-#pragma unroll
-            for (int p = 0; p < S; ++p) {
-                v4i w;
-                w[0] = (int)pack4(dg[p][0], dg[p][1], dg[p][2], dg[p][3]);
-                w[1] = (int)pack4(dg[p][4], dg[p][5], dg[p][6], dg[p][7]);
-                w[2] = (int)pack4(dg[p][8], dg[p][9], dg[p][10], dg[p][11]);
-                w[3] = (int)pack4(dg[p][12], dg[p][13], dg[p][14], dg[p][15]);
-                band[kp * S + p][s] = w;
-            }
+            for (int p = 0; p < S; ++p) band[kp * S + p][s] = dg[p];
         }
     }
     __syncthreads();

@@ -44,29 +44,6 @@ __device__ __forceinline__ int round_fixed(float x, const RowScale& rs) {
     return min(max(X, -rs.lim), rs.lim);
 }
 
-// Four bytes (low byte of each argument) packed little-endian with v_perm_b32.
-__device__ __forceinline__ uint32_t pack4(int b0, int b1, int b2, int b3) {
-    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b1, (uint32_t)b0, 0x0c0c0400u);
-    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)b3, (uint32_t)b2, 0x0c0c0400u);
-    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-}
-
-// The base-128 digits of a fixed-point value X (|X| <= 127 * 128^(S-1)), most significant
-// first: X = sum_p d[p] 128^(S-1-p) with a signed top digit d[0] = floor(X / 128^(S-1)) in
-// [-127, 127] and unsigned lower digits d[p] in [0, 127] (the bit fields of X). Any digit split
-// with these weights gives the same exact products; this one keeps the lower digits' sign bits
-// clear, which lowers the matrix cores' switching power (about 2% more int8 MFMA throughput
-// measured on MI355X with N(0,1) digit planes than balanced digits in [-64, 63]).
-template <int S>
-__device__ __forceinline__ void digits_of(int X, int (&d)[S]) {
-#pragma unroll
-    for (int p = S - 1; p >= 1; --p) {
-        d[p] = X & 127;
-        X >>= 7;  // arithmetic: floor(X / 128)
-    }
-    d[0] = X;
-}
-
 // Largest |x| over a 64-lane wavefront, in every lane.
 __device__ __forceinline__ float wave_max(float m) {
 #pragma unroll

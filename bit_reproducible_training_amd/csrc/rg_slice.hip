@@ -14,6 +14,7 @@
 //                  fixed-point integer of the definition and writes its S int8 digits
 //                  straight into the MFMA operand panel (1 KiB per digit and wavefront).
 // Max is exact and order-free, so the chunking never changes a bit.
+#include "rg_digits.h"
 #include "rg_internal.h"
 #include "repro_gemm_math.h"
 
@@ -311,7 +312,7 @@ __global__ void __launch_bounds__(256) absmax_kernel(SliceDesc a, SliceDesc b) {
 }
 
 // Rounds 16 values and writes them: S digit planes of 16 bytes (base 128, most significant
-// first, digits_of: X = sum_p d_p 128^(S-1-p), |d_0| <= 127, d_p in [0, 127] for p > 0), or
+// first, pack_word: X = sum_p d_p 128^(S-1-p), |d_0| <= 127, d_p in [0, 127] for p > 0), or
 // 16 int32 fixed-point values for INT32_OUT.
 template <int S, bool INT32_OUT>
 __device__ __forceinline__ void emit_panel(const SliceDesc& d, const float (&x)[16], const RowScale& rs,
@@ -325,21 +326,12 @@ __device__ __forceinline__ void emit_panel(const SliceDesc& d, const float (&x)[
         for (int q = 0; q < 4; ++q) o[q] = make_int4(X[4 * q], X[4 * q + 1], X[4 * q + 2], X[4 * q + 3]);
         return;
     }
-    int dg[S][16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        int d[S];
-        digits_of<S>(X[j], d);
-#pragma unroll
-        for (int p = 0; p < S; ++p) dg[p][j] = d[p];
-    }
+    v4i dg[S];
+    pack16<S>(X, dg);
     const int npk = d.Kp / PANEL_K;
-    uint4* o = reinterpret_cast<uint4*>(d.out) + ((size_t)rp * npk + kp) * S * (PANEL_BYTES / 16) + lane;
+    v4i* o = reinterpret_cast<v4i*>(d.out) + ((size_t)rp * npk + kp) * S * (PANEL_BYTES / 16) + lane;
 #pragma unroll
-    for (int p = 0; p < S; ++p)
-        o[(size_t)p * (PANEL_BYTES / 16)] =
-            make_uint4(pack4(dg[p][0], dg[p][1], dg[p][2], dg[p][3]), pack4(dg[p][4], dg[p][5], dg[p][6], dg[p][7]),
-                       pack4(dg[p][8], dg[p][9], dg[p][10], dg[p][11]), pack4(dg[p][12], dg[p][13], dg[p][14], dg[p][15]));
+    for (int p = 0; p < S; ++p) o[(size_t)p * (PANEL_BYTES / 16)] = dg[p];
 }
 
 // The 16 values of lane (half h) of panel kp in the row whose element k = 0 is at rowp (null
@@ -780,17 +772,14 @@ __device__ __forceinline__ void slice_onepass(const SliceDesc& d, long long blk)
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
-        int dg[S][4];
+        int X[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int d[S];
-            digits_of<S>(round_fixed(x[j], rs), d);
-#pragma unroll
-            for (int p = 0; p < S; ++p) dg[p][j] = d[p];
-        }
+        for (int j = 0; j < 4; ++j) X[j] = round_fixed(x[j], rs);
+        v4i dg[S];
+        pack_word<S>(X, dg, 0);
         uint32_t* o = o0 + (size_t)kp * S * (PANEL_BYTES / 4);
 #pragma unroll
-        for (int p = 0; p < S; ++p) o[p * (PANEL_BYTES / 4)] = pack4(dg[p][0], dg[p][1], dg[p][2], dg[p][3]);
+        for (int p = 0; p < S; ++p) o[p * (PANEL_BYTES / 4)] = (uint32_t)dg[p][0];
     }
 }
 
@@ -1180,17 +1169,14 @@ __device__ __forceinline__ void pslice_rows(const SliceDesc& d, long long blk) {
         const int kp = kp0 + i;
         if (kp >= npk) break;
         const float x[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-        int dg[S][4];
+        int X[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int dd[S];
-            digits_of<S>(round_fixed(x[j], rs), dd);
-#pragma unroll
-            for (int p = 0; p < S; ++p) dg[p][j] = dd[p];
-        }
+        for (int j = 0; j < 4; ++j) X[j] = round_fixed(x[j], rs);
+        v4i dg[S];
+        pack_word<S>(X, dg, 0);
         uint32_t* o = o0 + (size_t)kp * S * (PANEL_BYTES / 4);
 #pragma unroll
-        for (int p = 0; p < S; ++p) o[p * (PANEL_BYTES / 4)] = pack4(dg[p][0], dg[p][1], dg[p][2], dg[p][3]);
+        for (int p = 0; p < S; ++p) o[p * (PANEL_BYTES / 4)] = (uint32_t)dg[p][0];
     }
 }
 
