@@ -517,7 +517,7 @@ def widened(torch, rg, cpu=True, threads=16):
             pass_ = {"fwd": RC.FORWARD, "dW": RC.GRAD_WEIGHT, "dX": RC.GRAD_INPUT}[kind]
             algo = RC.conv2d_algo(pass_, g)
             row[kind + "_algo"] = "direct" if algo == RC.ALGO_DIRECT else "gemm"
-            if algo == RC.ALGO_DIRECT:  # the GEMM pipeline on the same inputs, for comparison
+            if algo == RC.ALGO_DIRECT:  # the MFMA route on the same inputs, for comparison
                 gws = torch.empty(max(RC.conv2d_algo_workspace(pass_, g, 3, RC.ALGO_GEMM), 1),
                                   dtype=torch.uint8, device="cuda")
                 o2 = torch.empty_like(o)
@@ -536,7 +536,7 @@ def widened(torch, rg, cpu=True, threads=16):
                                              ("dX", dy.cpu().numpy(), w.cpu().numpy())], outs))
     line["conv"] = convs
     # A ResNet-sized layer (batch 32, 64 -> 64 channels, 56 x 56, 3 x 3, padding 1): all three
-    # passes take the GEMM pipeline (forward on the implicit im2col matrix). GPU time and the
+    # passes take the implicit GEMMs that round the gathered values themselves. GPU time and the
     # same bits on a repeat; no CPU check at this size.
     g = rg.ConvShape(32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1)
     x = torch.randn(g.N, g.C, g.H, g.W, device="cuda")

@@ -50,12 +50,6 @@ constexpr size_t ALIGN = 256;
 size_t align_up(size_t x) { return (x + ALIGN - 1) / ALIGN * ALIGN; }
 int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 
-__device__ __forceinline__ uint32_t wave_umax(uint32_t m) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-    return m;
-}
-
 // Taps along one axis whose windows read source coordinate v: bit k for (v + pad - k) = s * o, 0 <= o < n.
 __device__ __forceinline__ uint32_t tap_mask(int v, int pad, int taps, int s, const FastDiv& ds, int n) {
     uint32_t m = 0;

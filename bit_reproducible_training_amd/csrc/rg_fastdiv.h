@@ -18,8 +18,7 @@ struct FastDiv {
 };
 
 inline FastDiv make_fastdiv(uint32_t d) {  // d >= 1
-    int l = 0;
-    while ((1ull << l) < d) ++l;
+    const int l = d > 1 ? 32 - __builtin_clz(d - 1) : 0;
     const uint64_t m = (((1ull << 32) * ((1ull << l) - d)) / d) + 1;
     return FastDiv{d, (uint32_t)m, l};
 }

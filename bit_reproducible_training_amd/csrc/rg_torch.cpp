@@ -133,16 +133,19 @@ Tensor gemm_run(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S
 
 Tensor gemm_ex(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S, int split_k,
                int tile_m, int tile_n, int algo, c10::optional<Tensor> out) {
-    return gemm_run(A, B, M, N, K, ta, tb, S, split_k, tile_m, tile_n, algo, out, c10::nullopt);
+    return gemm_run(std::move(A), std::move(B), M, N, K, ta, tb, S, split_k, tile_m, tile_n, algo,
+                    std::move(out), c10::nullopt);
 }
 
 // y[M, N] = x[M, K] w[N, K]^T, plus bias (or None).
 Tensor linear(Tensor x, Tensor w, c10::optional<Tensor> bias, int M, int N, int K, int S) {
-    return gemm_run(x, w, M, N, K, false, true, S, 1, 16, 16, RG_ALGO_AUTO, c10::nullopt, bias);
+    return gemm_run(std::move(x), std::move(w), M, N, K, false, true, S, 1, 16, 16, RG_ALGO_AUTO,
+                    c10::nullopt, std::move(bias));
 }
 
 Tensor gemm(Tensor A, Tensor B, int M, int N, int K, bool ta, bool tb, int S) {
-    return gemm_ex(A, B, M, N, K, ta, tb, S, 1, 16, 16, RG_ALGO_AUTO, c10::nullopt);
+    return gemm_run(std::move(A), std::move(B), M, N, K, ta, tb, S, 1, 16, 16, RG_ALGO_AUTO, c10::nullopt,
+                    c10::nullopt);
 }
 
 // out[b] = exact sum over a, c of x[a, b, c], rounded once; divided by A * C if mean
@@ -178,7 +181,7 @@ Tensor sum_run(Tensor x, int A, int B, int C, bool mean, c10::optional<Tensor> f
 }
 
 Tensor exact_sum(Tensor x, int A, int B, int C, bool mean) {
-    return sum_run(x, A, B, C, mean, c10::nullopt, 0);
+    return sum_run(std::move(x), A, B, C, mean, c10::nullopt, 0);
 }
 
 void require_flag(const Tensor& flag, const Tensor& x, const char* op) {
@@ -191,7 +194,7 @@ void require_flag(const Tensor& flag, const Tensor& x, const char* op) {
 Tensor exact_sum_watch(Tensor x, int A, int B, int C, Tensor flag, int op_id) {
     require_f32(x, "x");
     require_flag(flag, x, "exact_sum_watch");
-    return sum_run(x, A, B, C, false, flag, op_id);
+    return sum_run(std::move(x), A, B, C, false, std::move(flag), op_id);
 }
 
 repro_conv::ConvShape shape_of(const std::vector<int64_t>& x_shape, int F, int KH, int KW, int SY,
@@ -263,7 +266,7 @@ Tensor conv2d_bias(Tensor x, Tensor w, c10::optional<Tensor> bias, int SY, int S
 }
 
 Tensor conv2d(Tensor x, Tensor w, int SY, int SX, int PY, int PX, int S) {
-    return conv2d_bias(x, w, c10::nullopt, SY, SX, PY, PX, S);
+    return conv2d_bias(std::move(x), std::move(w), c10::nullopt, SY, SX, PY, PX, S);
 }
 
 // dW[F][C][KH][KW] from dY[N][F][OH][OW] and x (bindings.cpp:133-152).

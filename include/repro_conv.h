@@ -74,8 +74,8 @@ int rg_conv2d_grad_input_ws(const float* dy, const float* weight, float* dx,
 /* Diagnostic hooks, with no counterpart in the reference: a pass run with its algorithm
  * forced, for tests and benchmarks. pass: RG_CONV_FORWARD (a = x, b = weight),
  * RG_CONV_GRAD_WEIGHT (a = dy, b = x) or RG_CONV_GRAD_INPUT (a = dy, b = weight). algo:
- * RG_CONV_ALGO_AUTO (the choice of the entry points above), RG_CONV_ALGO_GEMM (im2col and the
- * int8 MFMA GEMM pipeline) or RG_CONV_ALGO_DIRECT (forward and input gradient only, while one
+ * RG_CONV_ALGO_AUTO (the choice of the entry points above), RG_CONV_ALGO_GEMM (the int8
+ * MFMA route) or RG_CONV_ALGO_DIRECT (forward and input gradient only, while one
  * sum has at most 2048 products and, forward, F*C*KH*KW <= 4096; else 801). Both algorithms
  * give the same bits. rg_conv2d_algo reports what AUTO resolves to; errors as above, plus 1 for
  * an unknown pass or algo. */
