@@ -40,15 +40,15 @@ STEADY_STEPS = 50
 # slicing launches (the slot marking and the one-read slicing), from rocprofv3 FETCH_SIZE /
 # WRITE_SIZE scaled by the same counters on a
 # 256 MiB device copy (profiles/contract_mfma_4096cube_traffic.md), each measured on the sources
-# whose SHA-256 (sources_digest) is given: the kernel file and rg_internal.h, which holds the
-# block order and the rounding helpers. A counter value cannot be read from inside this process,
-# so a figure is reported only while its sources are unchanged; otherwise it is null.
+# whose SHA-256 (sources_digest) is given: the kernel file and the headers that hold the block
+# order, the rounding helpers, the digits and the MFMA wrappers. A counter value cannot be read
+# from inside this process, so a figure is reported only while its sources are unchanged; otherwise it is null.
 CSRC = os.path.join(REPO, "bit_reproducible_training_amd", "csrc")
 TRAFFIC = {
-    "contract": (671606784, ("rg_contract.hip", "rg_internal.h"),
-                 "aad6c405111935b53b5551a3876ec8e399399485b748e7b6e9606e5651ad0bf0"),
-    "slicing": (235601510, ("rg_slice.hip", "rg_internal.h"),
-                "a762ab26f759129cac13e138d0c181325da016b9360adccd2312f5678f9aaeb8"),
+    "contract": (671575240, ("rg_contract.hip", "rg_internal.h", "rg_digits.h", "rg_mfma.h"),
+                 "928f2bec4bb4f70baebee00ecbad20b3f3a0eeb78f962178086fa61885a86197"),
+    "slicing": (235603489, ("rg_slice.hip", "rg_internal.h", "rg_digits.h"),
+                "0b4fdbb3b3b4853ad503bdc61b6173fca2ba2e76e25c970930c72537eb804157"),
 }
 FIXTURE = os.path.join(REPO, "tests", "golden", "baseline_configs.json")
 
@@ -1045,7 +1045,7 @@ def main():
                      "traffic": contract_traffic,
                      "traffic_source": "rocprofv3 FETCH_SIZE + WRITE_SIZE per launch, scaled by a "
                                        "256 MiB copy (profiles/contract_mfma_4096cube_traffic.md); "
-                                       "null when rg_contract.hip or rg_internal.h differs from the "
+                                       "null when one of its source files differs from the "
                                        "measured sources",
                      "kernel": "contract_mfma<3,2,1,2,4>: int8 ops = 9 * 2MNK per launch, one "
                                "launch per step; achieved = ops / HIP-event duration"},
