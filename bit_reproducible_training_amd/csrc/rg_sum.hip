@@ -6,9 +6,11 @@
 // units, and every partial sum is exact while h - l + ceil(log2 n) <= 29: a thread keeps the largest
 // magnitude and the smallest non-zero one of what its binary64 sum holds (16 values at a time), and
 // when the next 16 would break the bound it moves the sum into its superaccumulator and starts
-// again; 16 values that break it by themselves go into the superaccumulator one by one. N(0, 1)
-// data never does either within a thread's share. A value costs about five vector instructions
-// (widening, addition, the two bounds) instead of a read-modify-write of LDS.
+// again; 16 values that break it by themselves go into the superaccumulator, and the binary64 sum
+// stays. N(0, 1) data hardly does either within a thread's share: a value costs about five vector
+// instructions (widening, addition, the two bounds). Gradients of a softmax cross-entropy do both all
+// the time (probabilities down to 1e-9 next to one near 1), so the superaccumulator's additions have
+// no branch and return nothing: about 14 vector instructions and one LDS addition a value.
 //
 // The superaccumulator is exact for every float: 10 limbs per thread in LDS (limb l of thread t at
 // acc[l][t], radix 2^32, limb l weighing 2^(32 l - 149)), cleared when a thread first needs it. A
@@ -32,7 +34,10 @@
 // 87 -> 37 (5.6 TB/s), 8192 x 4096 rows 45 -> 25 (5.3 TB/s) and columns 56 -> 28, 16384 rows of 1024
 // 34 -> 14.5, 65536 rows of 128 86 -> 27, 1000 x 33 x 7 27 -> 5, one sum of 2^24 values 38 -> 23 (the
 // merge of its 2048 chunks is one block's). The large ones run at the rate of a copy's reads; small
-// ones are two launches.
+// ones are two launches. That is N(0, 1) data; values over a wide range (a softmax gradient, and
+// uniform exponents in +-20): 8192 x 3072 columns 49 -> 43 and 49 -> 38, 256 x 64 x 3136 87 -> 58 and
+// 87 -> 52. (One by one, with their history moved out first, the values that do not fit took 94, 82,
+// 177 and 146.)
 #include "rg_fastdiv.h"
 #include "rg_internal.h"
 #include "repro_sum.h"
@@ -61,15 +66,20 @@ struct LdsAcc {
 #pragma unroll
         for (int l = 0; l < LIMBS; ++l) p[l * SUM_THREADS] = 0;
     }
-    __device__ void add(float x, int& nonfinite) {
-        int idx;
-        uint64_t v;
-        bool neg;
-        if (!repro_sum::wide_term(x, idx, v, neg)) {
-            nonfinite = 1;
-            return;
-        }
-        p[idx * SUM_THREADS] += neg ? -(int64_t)v : (int64_t)v;
+    // One value, by an LDS addition that returns nothing (nobody else touches the address, so it is
+    // atomic for free and nothing waits for it): p[idx] += +-significand << s. The exponent of a NaN
+    // or an infinity is 255, which the caller looks for in the largest one (top_e); what it adds is
+    // in bounds and never used.
+    __device__ __forceinline__ void add(float x, uint32_t& top_e) {
+        const uint32_t b = __float_as_uint(x), e = (b >> 23) & 0xFFu;
+        top_e = max(top_e, e);
+        const uint32_t sig = (b & 0x7FFFFFu) | (min(e, 1u) << 23), sh = max(e, 1u) - 1u;
+        const int32_t sign = (int32_t)b >> 31;  // 0 or -1
+        const int64_t v = ((int32_t)sig ^ sign) - sign;
+        bump(sh >> 5, (int64_t)((uint64_t)v << (sh & 31u)));
+    }
+    __device__ __forceinline__ void bump(uint32_t limb, int64_t v) {
+        __hip_atomic_fetch_add(p + limb * SUM_THREADS, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     // An exact sum of floats held in binary64 (a multiple of 2^-149 below 2^159): its 53-bit
     // significand, shifted to a limb boundary, is three 32-bit terms.
@@ -91,9 +101,9 @@ struct LdsAcc {
         const int64_t t0 = (int64_t)(uint32_t)(m << s);
         const int64_t t1 = (int64_t)(uint32_t)(m >> (32 - s)), t2 = s ? (int64_t)(m >> (64 - s)) : 0;
         const int64_t sign = (int64_t)b >> 63;  // 0 or -1
-        p[idx * SUM_THREADS] += (t0 ^ sign) - sign;
-        p[(idx + 1) * SUM_THREADS] += (t1 ^ sign) - sign;
-        p[(idx + 2) * SUM_THREADS] += (t2 ^ sign) - sign;
+        bump(idx, (t0 ^ sign) - sign);
+        bump(idx + 1, (t1 ^ sign) - sign);
+        bump(idx + 2, (t2 ^ sign) - sign);
     }
     // Carries: limbs 0..LIMBS-2 into [0, 2^32), the top limb keeps the sign.
     __device__ void carry() {
@@ -116,7 +126,9 @@ __device__ __forceinline__ int log2_up(uint32_t n) { return 32 - __clz((int)(n -
 // Whether n values with largest magnitude `top` and smallest non-zero one `low` sum exactly in
 // binary64 in any order: h - l + ceil(log2 n) <= 29. low is kept as 2 * bits - 1 without the sign
 // (zeros map to the largest key, so they never are the smallest); a subnormal counts as the smallest
-// normal exponent, whose last bit is its unit. An infinity fails the bound.
+// normal exponent, whose last bit is its unit. An infinity may pass the bound (with magnitudes near
+// 2^100 and above beside it), and a NaN is in neither: the binary64 sum is not finite then, which every
+// use of it checks.
 __device__ __forceinline__ bool sums_exactly(float top, uint32_t low, int log2n) {
     const int h = (int)(__float_as_uint(top) >> 23), l = max(1, (int)(low >> 24));
     return max(h, 1) - l + log2n <= 29;
@@ -134,10 +146,7 @@ struct ThreadSum {
     int nonfinite = 0;
 
     __device__ void spill() {    // binary64 -> limbs
-        if (!used) {
-            limbs.clear();
-            used = true;
-        }
+        use();
         limbs.add_double(acc0 + acc1, nonfinite);
         ++since;
         acc0 = acc1 = 0.0;
@@ -145,46 +154,46 @@ struct ThreadSum {
         low = 0xFFFFFFFFu;
         count = 0;
     }
+    __device__ void use() {
+        if (!used) {
+            limbs.clear();
+            used = true;
+        }
+    }
     template <int N>
     __device__ __forceinline__ void add(const float (&v)[N]) {
         // A NaN is in neither bound; it makes the binary64 sum a NaN, which spill() and the final
         // steps see.
-        float m = top;
-        uint32_t k = low;
+        float m = 0.0f;
+        uint32_t k = 0xFFFFFFFFu;
 #pragma unroll
         for (int i = 0; i < N; ++i) m = fmaxf(m, __builtin_fabsf(v[i]));
 #pragma unroll
         for (int i = 0; i < N; ++i) k = min(k, 2u * __float_as_uint(v[i]) - 1u);
-        if (__builtin_expect(!sums_exactly(m, k, log2_up(count + N)), 0)) {
-            spill();
+        const float m_all = fmaxf(top, m);
+        const uint32_t k_all = min(low, k);
+        if (__builtin_expect(!sums_exactly(m_all, k_all, log2_up(count + N)), 0)) {
+            const bool alone = sums_exactly(m, k, log2_up(N));
+            if (alone) {
+                spill();
+                top = m;
+                low = k;
+            } else {  // (what the binary64 sum holds stays there)
+                use();
+                uint32_t top_e = 0;
 #pragma unroll
-            for (int i = 0; i < N; ++i) top = fmaxf(top, __builtin_fabsf(v[i]));
-#pragma unroll
-            for (int i = 0; i < N; ++i) low = min(low, 2u * __float_as_uint(v[i]) - 1u);
-            if (!sums_exactly(top, low, log2_up(N))) {
-#pragma unroll 1
-                for (int i = 0; i < N; ++i) {
-                    float x = v[0];
-#pragma unroll
-                    for (int j = 1; j < N; ++j) x = i == j ? v[j] : x;
-                    limbs.add(x, nonfinite);
-                }
+                for (int i = 0; i < N; ++i) limbs.add(v[i], top_e);
+                nonfinite |= top_e == 0xFFu;
                 since += N;
-                top = 0.0f;
-                low = 0xFFFFFFFFu;
-                if (since >= FLUSH_AT - BATCH) {
-                    limbs.carry();
-                    since = 0;
-                }
-                return;
             }
             if (since >= FLUSH_AT - BATCH) {
                 limbs.carry();
                 since = 0;
             }
+            if (!alone) return;
         } else {
-            top = m;
-            low = k;
+            top = m_all;
+            low = k_all;
         }
         count += N;
 #pragma unroll
@@ -200,8 +209,6 @@ struct ThreadSum {
     }
 };
 
-// C == 1. Block = 64 outputs (lanes) x 4 row phases (waves); chunk = blockIdx.y covers rows
-// [a0, a1), phase w takes rows a0 + w, a0 + w + 4, ...
 // Lowers flag[0] to op_id if any of the wave's lanes holds `bad`: one atomic per such wave.
 __device__ inline void report(bool bad, int* flag, int op_id) {
     const unsigned long long votes = __ballot(bad);
@@ -209,7 +216,7 @@ __device__ inline void report(bool bad, int* flag, int op_id) {
         atomicMin(flag, op_id);
 }
 
-// watch (in this kernel and the next): the pass that reads the values also reports a NaN or an
+// watch (in both kernels below): the pass that reads the values also reports a NaN or an
 // infinity among them, as scan_nonfinite does (watch.flag null: no report). A bias gradient and the
 // check of the incoming gradient are then one read of it: 8192 x 3072, 17 us of scan saved.
 struct Watch {
@@ -217,6 +224,8 @@ struct Watch {
     int op_id;
 };
 
+// C == 1. Block = 64 outputs (lanes) x 4 row phases (waves); chunk = blockIdx.y covers rows
+// [a0, a1), phase w takes rows a0 + w, a0 + w + 4, ...
 __global__ void __launch_bounds__(SUM_THREADS)
 sum_columns(const float* __restrict__ x, int A, int B, int rows_per_chunk, int chunks,
             uint32_t divisor, float* __restrict__ out, int64_t* __restrict__ part,

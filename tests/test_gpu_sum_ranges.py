@@ -65,3 +65,56 @@ def test_sum_of_nonfinite_values_is_nan(torch_gpu, special):
             got = bits(rg.exact_sum(to_dev(torch_gpu, x.ravel()), A, B, C))
             want = O.exact_sum(x.ravel(), A, B, C).view(np.uint32)
             assert np.array_equal(got, want) and np.isnan(want.view(np.float32)[B // 2])
+
+
+@pytest.mark.parametrize("kind", ["softmax", "wild", "mixed"])
+def test_long_sums_of_values_that_leave_binary64(torch_gpu, kind):
+    """One chunk, so that a thread's share takes hundreds of batches: the superaccumulator resolves
+    its carries many times, between batches that fit binary64 and batches that do not."""
+    for A, B, C in ((60000, 3, 1), (1, 2, 90001), (4, 2, 20000)):
+        rng = np.random.default_rng(A + C)
+        x = _values("wild" if kind == "wild" else "spread13", A * B * C, rng)
+        if kind == "softmax":
+            x = np.exp(x / np.abs(x).max() * 40.0 - 40.0).astype(np.float32)
+        elif kind == "mixed":  # runs of 4096 values of one magnitude, some of them with outliers
+            x *= (2.0 ** (np.arange(x.size) // 4096 * 37 % 120 - 60)).astype(np.float32)
+            x[::2999] = np.float32(3.0e38)
+        for mean in (False, True):
+            note("long sum", kind, (A, B, C), mean)
+            cfg = rg.SumConfig(chunks=1, mean=mean)
+            dx, out = to_dev(torch_gpu, x), torch_gpu.empty(B, device="cuda")
+            ws = torch_gpu.empty(max(rg.make_sum_plan(A, B, C, cfg).workspace_bytes, 1), dtype=torch_gpu.uint8,
+                                 device="cuda")
+            assert rg.repro_sum_fp32_ws(dx.data_ptr(), out.data_ptr(), A, B, C, cfg, ws.data_ptr(), ws.numel(),
+                                        torch_gpu.cuda.current_stream().cuda_stream) == 0
+            want = O.exact_sum(x, A, B, C, mean)
+            assert np.array_equal(bits(out), want.view(np.uint32)), (kind, A, B, C, mean)
+
+
+def test_wide_ranges_cost_little_more(torch_gpu):
+    """Values that do not fit binary64 together cost at most 2.5 times as much as N(0, 1) ones (1.4-1.8
+    measured; adding them one by one took 3.3-4.7 times as long)."""
+    torch = torch_gpu
+    torch.manual_seed(1)
+
+    def fastest(x, shape):
+        times = []
+        for _ in range(8):
+            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            ev[0].record()
+            for _ in range(20):
+                rg.exact_sum(x, *shape)
+            ev[1].record()
+            torch.cuda.synchronize()
+            times.append(ev[0].elapsed_time(ev[1]))
+        return min(times)
+
+    for shape in ((8192, 3072, 1), (256, 64, 3136)):
+        x = torch.randn(*shape, device="cuda")
+        wide = x * torch.exp2(torch.randint(-20, 21, shape, device="cuda").float())
+        p = torch.softmax(4 * x.view(shape[0], -1), 1)
+        p[:, 0] -= 1
+        note("sum cost", shape)
+        plain = fastest(x, shape)
+        for y in (wide, p / shape[0]):
+            assert fastest(y, shape) < 2.5 * plain, shape
