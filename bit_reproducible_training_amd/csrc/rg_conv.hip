@@ -718,7 +718,8 @@ struct ConvPlan {
 
 int conv_plan(Kind kind, const rg_conv_shape* s, int S, int algo, ConvPlan* P) {
     if (!valid(s, S)) return hipErrorInvalidValue;
-    if (algo != RG_CONV_ALGO_AUTO && algo != RG_CONV_ALGO_GEMM && algo != RG_CONV_ALGO_DIRECT)
+    if (algo != RG_CONV_ALGO_AUTO && algo != RG_CONV_ALGO_GEMM && algo != RG_CONV_ALGO_DIRECT &&
+        algo != RG_CONV_ALGO_PIPELINE && algo != RG_CONV_ALGO_FUSED)
         return hipErrorInvalidValue;
     ConvPlan p;
     std::memset(&p, 0, sizeof p);
@@ -736,24 +737,26 @@ int conv_plan(Kind kind, const rg_conv_shape* s, int S, int algo, ConvPlan* P) {
         *P = p;
         return hipSuccess;
     }
-    {
+    if (algo != RG_CONV_ALGO_PIPELINE) {
         DeviceInfo dev;
         const int e = query_device(&dev);
         if (e != hipSuccess) return e;
         if (!dev.gfx950) return hipErrorNotSupported;
+        const bool forced = algo == RG_CONV_ALGO_FUSED;
         if (kind == Kind::GradWeight) {
-            if (dw_plan(*s, S, dev.num_cus, &p.d)) {
+            if (dw_plan(*s, S, dev.num_cus, forced, &p.d)) {
                 p.dwfused = true;
                 p.total = p.d.total;
                 *P = p;
                 return hipSuccess;
             }
-        } else if (fused_plan((int)kind, *s, S, dev.num_cus, &p.f)) {
+        } else if (fused_plan((int)kind, *s, S, dev.num_cus, forced, &p.f)) {
             p.fused = true;
             p.total = p.f.total;
             *P = p;
             return hipSuccess;
         }
+        if (forced) return hipErrorNotSupported;
     }
     rg_config cfg;
     rg_config_init(&cfg);
@@ -1035,7 +1038,7 @@ int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int
     for (int i = 0; i < 8; ++i) info[i] = 0;
     if (pass == RG_CONV_GRAD_WEIGHT) {
         rg::DwPlan d;
-        if (!rg::dw_plan(*g, S, num_cus, &d)) return hipSuccess;
+        if (!rg::dw_plan(*g, S, num_cus, false, &d)) return hipSuccess;
         info[0] = info[1] = 1;
         info[2] = d.parts;
         info[3] = d.RC;
@@ -1046,7 +1049,7 @@ int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int
         return hipSuccess;
     }
     rg::FusedPlan p;
-    if (!rg::fused_plan(pass, *g, S, num_cus, &p)) return hipSuccess;
+    if (!rg::fused_plan(pass, *g, S, num_cus, false, &p)) return hipSuccess;
     info[0] = 1;
     info[1] = p.patch;
     info[2] = p.split;

@@ -29,8 +29,9 @@ struct DwPlan {
     size_t xmax, dmax, ea, eb, part, total;  // workspace offsets
 };
 
-// Fills *plan and returns true when the fused kernels take this weight gradient (a valid shape).
-bool dw_plan(const rg_conv_shape& s, int S, int num_cus, DwPlan* plan);
+// Fills *plan and returns true when the fused kernels take this weight gradient (a valid shape): where
+// they are faster than the GEMM pipeline, or with `forced` wherever they can.
+bool dw_plan(const rg_conv_shape& s, int S, int num_cus, bool forced, DwPlan* plan);
 
 int dw_launch(const DwPlan& p, const float* dy, const float* x, float* dw, char* ws, hipStream_t stream);
 

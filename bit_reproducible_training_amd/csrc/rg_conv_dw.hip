@@ -543,7 +543,7 @@ void launch_s(const DwPlan& p, const float* dy, const float* x, char* ws, hipStr
 
 }  // namespace
 
-bool dw_plan(const rg_conv_shape& s, int S, int num_cus, DwPlan* out) {
+bool dw_plan(const rg_conv_shape& s, int S, int num_cus, bool forced, DwPlan* out) {
     DwPlan p;
     std::memset(&p, 0, sizeof p);
     p.S = S; p.N = s.N; p.C = s.C; p.H = s.H; p.W = s.W; p.F = s.F;
@@ -583,7 +583,7 @@ bool dw_plan(const rg_conv_shape& s, int S, int num_cus, DwPlan* out) {
         }
         if (p.NS && ns >= 2 * p.NS) break;
     }
-    if (!p.NS || best < 0.4) return false;
+    if (!p.NS || (best < 0.4 && !forced)) return false;
     p.PH = (p.OH - 1) * p.SY + p.TH;
     const double vrows = (double)p.N * p.NS * p.OH;
     if (vrows * (p.SY + p.TH) >= 1073741824.0) return false;
@@ -620,7 +620,7 @@ bool dw_plan(const rg_conv_shape& s, int S, int num_cus, DwPlan* out) {
     const double gemm = 24.0 + 3.0e-4 * windows + (18.0 * windows * p.K + 12.0 * windows * p.F) / 4.5e6 +
                         2.0 * windows * p.F * p.K * (S * S / 9.0) / 2.2e8;
     const double here = 8.0 + 4.0 * ((double)p.N * p.C * p.H * p.W + windows * p.F) / 5.0e6 + cost;
-    if (here > 0.88 * gemm) return false;
+    if (here > 0.88 * gemm && !forced) return false;
     // Maxima: enough blocks to keep the memory busy.
     p.pgroups = ceil_div((long long)p.H * p.W, DW_PIX);
     p.xgroups = (int)std::max<long long>(1, std::min<long long>(std::min(p.N, 64), ceil_div(2048, (long long)p.C * p.pgroups)));

@@ -61,8 +61,9 @@ struct FusedPlan {
 };
 
 // Fills *plan and returns true when the fused kernels take this pass (kind: RG_CONV_FORWARD or
-// RG_CONV_GRAD_INPUT; the shape is valid).
-bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, FusedPlan* plan);
+// RG_CONV_GRAD_INPUT; the shape is valid): where they are faster than the GEMM pipeline, or with
+// `forced` wherever they can.
+bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, bool forced, FusedPlan* plan);
 
 // a: x (forward) or dY; w: the layer's weights; bias: one float per output channel, added to the
 // rounded outputs, or null; out: y or dX.

@@ -947,7 +947,7 @@ fused_reduce(FusedPlan p, const char* __restrict__ ws, float* __restrict__ out,
 
 }  // namespace
 
-bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, FusedPlan* out) {
+bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, bool forced, FusedPlan* out) {
     FusedPlan p;
     std::memset(&p, 0, sizeof p);
     const int OH = (s.H + 2 * s.PY - s.KH) / s.SY + 1, OW = (s.W + 2 * s.PX - s.KW) / s.SX + 1;
@@ -1002,8 +1002,8 @@ bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, FusedPlan*
     if (dx) {
         const double here = (double)s.N * s.H * s.W * 32 * ceil_div(p.F, 32) * kpad / (s.SY * s.SX);
         const double gemm = (double)s.N * OH * OW * (64.0 * ceil_div(s.C * T, 64)) * (64.0 * ceil_div(s.F, 64));
-        if (here > 6.0 * gemm) return false;
-    } else if (kpad > (p.patch ? 2.25 : 1.5) * 64.0 * ceil_div(s.C * T, 64)) {
+        if (here > 6.0 * gemm && !forced) return false;
+    } else if (!forced && kpad > (p.patch ? 2.25 : 1.5) * 64.0 * ceil_div(s.C * T, 64)) {
         return false;
     }
     const int bf = 32 * p.tf * p.nwf;
@@ -1105,7 +1105,7 @@ bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, FusedPlan*
     // not at stride 1, so that every value is fetched and rounded once per tap (32 x 128 x 28 x 28,
     // 128 filters 3x3, stride 2: 35 against 44). Longer windows it packs first (32 x 512 x 7 x 7,
     // 512 filters: 81 against 66 here).
-    if (!dx && (p.split > 1 || (!p.patch && T > 1)) && s.C * T <= ONEPASS_MAX_K) return false;
+    if (!forced && !dx && (p.split > 1 || (!p.patch && T > 1)) && s.C * T <= ONEPASS_MAX_K) return false;
     p.dblocks = make_fastdiv((uint32_t)p.blocks);
     p.dOPL = make_fastdiv((uint32_t)p.OPL);
     p.dF = make_fastdiv((uint32_t)p.F);

@@ -88,10 +88,11 @@ def repro_conv2d_grad_input_ws(dy, weight, dx, g, S, workspace, workspace_bytes,
 
 
 # Passes and algorithms of the diagnostic hooks (include/repro_conv.h): AUTO is what the entry
-# points above choose, GEMM the im2col + MFMA GEMM pipeline, DIRECT the one-launch kernels for
-# small filters (forward and input gradient).
+# entry points above choose, GEMM the MFMA route (PIPELINE, im2col and the GEMM pipeline, or FUSED,
+# the implicit GEMMs, whichever is the faster), DIRECT the one-launch kernels for small filters
+# (forward and input gradient).
 FORWARD, GRAD_WEIGHT, GRAD_INPUT = 0, 1, 2
-ALGO_AUTO, ALGO_GEMM, ALGO_DIRECT = 0, 1, 2
+ALGO_AUTO, ALGO_GEMM, ALGO_DIRECT, ALGO_PIPELINE, ALGO_FUSED = 0, 1, 2, 3, 4
 
 
 def conv2d_algo(pass_, g, S=3):
@@ -135,7 +136,8 @@ def conv2d_grad_input(dy, w, x_shape, SY, SX, PY, PX, S=3):
                                       int(PY), int(PX), int(S))
 
 
-__all__ = ["ALGO_AUTO", "ALGO_DIRECT", "ALGO_GEMM", "FORWARD", "GRAD_INPUT", "GRAD_WEIGHT",
+__all__ = ["ALGO_AUTO", "ALGO_DIRECT", "ALGO_FUSED", "ALGO_GEMM", "ALGO_PIPELINE", "FORWARD",
+           "GRAD_INPUT", "GRAD_WEIGHT",
            "conv2d_algo", "conv2d_algo_workspace", "repro_conv2d_algo_ws",
            "ConvShape", "conv2d", "conv2d_grad_input", "conv2d_grad_weight",
            "conv2d_grad_input_workspace", "conv2d_grad_weight_workspace", "conv2d_workspace",

@@ -75,12 +75,16 @@ int rg_conv2d_grad_input_ws(const float* dy, const float* weight, float* dx,
  * forced, for tests and benchmarks. pass: RG_CONV_FORWARD (a = x, b = weight),
  * RG_CONV_GRAD_WEIGHT (a = dy, b = x) or RG_CONV_GRAD_INPUT (a = dy, b = weight). algo:
  * RG_CONV_ALGO_AUTO (the choice of the entry points above), RG_CONV_ALGO_GEMM (the int8
- * MFMA route) or RG_CONV_ALGO_DIRECT (forward and input gradient only, while one
- * sum has at most 2048 products and, forward, F*C*KH*KW <= 4096; else 801). Both algorithms
- * give the same bits. rg_conv2d_algo reports what AUTO resolves to; errors as above, plus 1 for
- * an unknown pass or algo. */
+ * MFMA route: the faster of the next two, as AUTO takes it), RG_CONV_ALGO_PIPELINE (im2col and the
+ * GEMM pipeline, any shape), RG_CONV_ALGO_FUSED (the implicit GEMMs that round the gathered values
+ * themselves; 801 for a shape they cannot take: input gradients with SY*SX > 4, weight gradients
+ * with SX > 2, kernels longer than 31, sums or offsets past their limits) or
+ * RG_CONV_ALGO_DIRECT (forward and input gradient only, while one sum has at most 2048 products and,
+ * forward, F*C*KH*KW <= 4096; else 801). All algorithms give the same bits. rg_conv2d_algo reports
+ * what AUTO resolves to, GEMM or DIRECT; errors as above, plus 1 for an unknown pass or algo. */
 enum { RG_CONV_FORWARD = 0, RG_CONV_GRAD_WEIGHT = 1, RG_CONV_GRAD_INPUT = 2 };
-enum { RG_CONV_ALGO_AUTO = 0, RG_CONV_ALGO_GEMM = 1, RG_CONV_ALGO_DIRECT = 2 };
+enum { RG_CONV_ALGO_AUTO = 0, RG_CONV_ALGO_GEMM = 1, RG_CONV_ALGO_DIRECT = 2,
+       RG_CONV_ALGO_PIPELINE = 3, RG_CONV_ALGO_FUSED = 4 };
 int rg_conv2d_algo(int pass, const rg_conv_shape* g, int S, int* algo);
 int rg_conv2d_algo_workspace(int pass, const rg_conv_shape* g, int S, int algo, size_t* bytes);
 int rg_conv2d_algo_ws(int pass, const float* a, const float* b, float* out, const rg_conv_shape* g,

@@ -138,3 +138,14 @@ def test_weight_gradient_slots_are_free_and_ready(steps):
         if c >= 4:  # tables 0 .. 3 are built before the first stage
             built = -(-(c - 3) * steps // 2)
             assert built + 1 <= c * steps // 2 - 2, (steps, c)
+
+
+def test_forced_algorithms_are_known():
+    g = rg.ConvShape(2, 3, 9, 9, 4, 3, 3)
+    for algo, known in ((3, True), (4, True), (5, False), (-1, False)):
+        try:
+            rg.repro_conv.conv2d_algo_workspace(FWD, g, 3, algo)
+            code = 0
+        except rg.ReproGemmError as e:
+            code = e.code
+        assert (code != 1) == known, algo  # (without a GPU a known one stops at the device query)

@@ -38,6 +38,20 @@ SHAPES = [
 ]
 
 
+# The window gather with several taps: strides, padding, one and several parts along k, channels off a
+# group of 16, taps beyond every source row, 31 taps a side.
+GATHERS = [
+    (1, 256, 9, 9, 70, 7, 7, 2, 2, 3, 3),
+    (1, 512, 7, 7, 40, 3, 3, 2, 2, 1, 1),
+    (1, 4200, 5, 5, 33, 1, 1, 1, 1, 0, 0),
+    (2, 20, 13, 17, 33, 5, 3, 3, 2, 2, 0),
+    (3, 5, 11, 9, 12, 3, 3, 2, 1, 1, 1),
+    (2, 16, 3, 40, 16, 31, 2, 1, 2, 15, 1),
+    (1, 33, 2, 2, 130, 5, 5, 1, 2, 2, 2),
+    (1, 18, 4, 140, 20, 1, 31, 1, 3, 0, 15),
+]
+
+
 def _inputs(shape, seed):
     N, C, H, W, F, KH, KW = shape[:7]
     OH, OW = O.conv_out_hw(shape)
@@ -51,7 +65,7 @@ def _inputs(shape, seed):
 def _check(torch, shape, S, x, w, dy):
     for kind, a, b in (("fwd", x, w), ("dX", dy, w), ("dW", dy, x)):
         note("fused conv", kind, shape, "S=%d" % S)
-        got = _run_algo(torch, kind, a, b, shape, S, RC.ALGO_GEMM).view(np.uint32).ravel()
+        got = _run_algo(torch, kind, a, b, shape, S, RC.ALGO_FUSED).view(np.uint32).ravel()
         assert np.array_equal(got, _oracle(kind, a, b, shape, S).view(np.uint32).ravel()), (kind, shape, S)
 
 
@@ -59,6 +73,17 @@ def _check(torch, shape, S, x, w, dy):
 def test_fused_matches_oracle(torch_gpu, S):
     for i, shape in enumerate(SHAPES):
         _check(torch_gpu, shape, S, *_inputs(shape, 10 * S + i))
+
+
+@pytest.mark.parametrize("S", [1, 2, 3])
+def test_gathered_taps_match_oracle(torch_gpu, S):
+    for i, shape in enumerate(GATHERS):
+        x, w, dy = _inputs(shape, 1000 + 10 * S + i)
+        if i % 2:
+            x[np.random.default_rng(i).integers(0, x.size, 4)] = [np.nan, np.inf, -np.inf, 1e-40]
+        note("fused gather", shape, "S=%d" % S)
+        got = _run_algo(torch_gpu, "fwd", x, w, shape, S, RC.ALGO_FUSED).view(np.uint32).ravel()
+        assert np.array_equal(got, _oracle("fwd", x, w, shape, S).view(np.uint32).ravel()), (shape, S)
 
 
 def test_shapes_cover_the_routes():
