@@ -162,6 +162,8 @@ _SIGNATURES = {
     "rg_conv2d_grad_input_ws": _CONV_RUN,
     "rg_test_conv_fused": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape), ctypes.c_int,
                                           ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
+    "rg_test_conv_plan": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape), ctypes.c_int,
+                                         ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
     "rg_conv2d_algo": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape), ctypes.c_int,
                                       ctypes.POINTER(ctypes.c_int)]),
     "rg_conv2d_algo_workspace": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape),

@@ -1033,12 +1033,15 @@ int rg_conv2d_algo_ws(int pass, const float* a, const float* b, float* out, cons
                         workspace_bytes, stream);
 }
 
-int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int* info) {
+int rg_test_conv_plan(int pass, const rg_conv_shape* g, int S, int num_cus, int forced, int* info) {
     if (!g || !info || !rg::valid_pass(pass) || !rg::valid(g, S) || num_cus < 1) return hipErrorInvalidValue;
-    for (int i = 0; i < 8; ++i) info[i] = 0;
+    for (int i = 0; i < 11; ++i) info[i] = 0;
     if (pass == RG_CONV_GRAD_WEIGHT) {
         rg::DwPlan d;
-        if (!rg::dw_plan(*g, S, num_cus, false, &d)) return hipSuccess;
+        if (!rg::dw_plan(*g, S, num_cus, forced != 0, &d)) return hipSuccess;
+        info[8] = d.KS;
+        info[9] = d.per_part;
+        info[10] = d.chunks;
         info[0] = info[1] = 1;
         info[2] = d.parts;
         info[3] = d.RC;
@@ -1049,7 +1052,10 @@ int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int
         return hipSuccess;
     }
     rg::FusedPlan p;
-    if (!rg::fused_plan(pass, *g, S, num_cus, false, &p)) return hipSuccess;
+    if (!rg::fused_plan(pass, *g, S, num_cus, forced != 0, &p)) return hipSuccess;
+    info[8] = p.cls[0].T;
+    info[9] = p.cls[0].stages;
+    info[10] = (p.C + 15) / 16;
     info[0] = 1;
     info[1] = p.patch;
     info[2] = p.split;
@@ -1059,6 +1065,14 @@ int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int
     info[6] = p.cls[0].pxgroups;
     info[7] = p.tf;
     return hipSuccess;
+}
+
+int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int* info) {
+    if (!info) return hipErrorInvalidValue;
+    int all[11];
+    const int e = rg_test_conv_plan(pass, g, S, num_cus, 0, all);
+    if (e == hipSuccess) std::copy(all, all + 8, info);
+    return e;
 }
 
 }  // extern "C"

@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "repro_gemm_math.h"
+#include "rg_conv_cost.h"
 #include "rg_digits.h"
 #include "rg_internal.h"
 #include "rg_mfma.h"
@@ -583,7 +584,7 @@ bool dw_plan(const rg_conv_shape& s, int S, int num_cus, bool forced, DwPlan* ou
         }
         if (p.NS && ns >= 2 * p.NS) break;
     }
-    if (!p.NS || (best < 0.4 && !forced)) return false;
+    if (!p.NS) return false;
     p.PH = (p.OH - 1) * p.SY + p.TH;
     const double vrows = (double)p.N * p.NS * p.OH;
     if (vrows * (p.SY + p.TH) >= 1073741824.0) return false;
@@ -609,23 +610,27 @@ bool dw_plan(const rg_conv_shape& s, int S, int num_cus, bool forced, DwPlan* ou
         }
     }
     if (tiles * p.parts >= 1073741824.0) return false;
-    // Against the GEMM pipeline, fitted to its times: seven launches and passes over long rows
-    // (0.3 us a thousand windows), its packing (18 bytes of traffic per window and position, 12 per
-    // value of dY) and contraction (220 TFLOP/s at S = 3). With many filters and few windows the
-    // pipeline is ahead, since it rounds every value once where this kernel rounds it once per block
-    // of filters (32 x 512 x 7 x 7, 512 filters: 69 us against 130 here; 8 x 256 x 14 x 14, 256
-    // filters: 50 against 53); most other shapes are 1.2-3 times faster here. The factor keeps the
-    // pipeline where the two are close.
-    const double windows = (double)p.N * p.OH * p.OW;
-    const double gemm = 24.0 + 3.0e-4 * windows + (18.0 * windows * p.K + 12.0 * windows * p.F) / 4.5e6 +
-                        2.0 * windows * p.F * p.K * (S * S / 9.0) / 2.2e8;
-    const double here = 8.0 + 4.0 * ((double)p.N * p.C * p.H * p.W + windows * p.F) / 5.0e6 + cost;
-    if (here > 0.88 * gemm && !forced) return false;
     // Maxima: enough blocks to keep the memory busy.
     p.pgroups = ceil_div((long long)p.H * p.W, DW_PIX);
     p.xgroups = (int)std::max<long long>(1, std::min<long long>(std::min(p.N, 64), ceil_div(2048, (long long)p.C * p.pgroups)));
     p.dgroups = (int)std::max<long long>(1, std::min<long long>(std::min(p.N, 64), ceil_div(1024, p.F)));
     if ((double)p.C * p.xgroups * p.pgroups + (double)p.F * p.dgroups >= 1073741824.0) return false;
+    if (!forced) {
+        // Against the GEMM pipeline (rg_conv_cost.h: how both were fitted, and what it replaced). With
+        // many filters and few windows the pipeline is ahead, since it rounds every value once where
+        // this kernel rounds it once per block of filters (32 x 512 x 7 x 7, 512 filters: 69 us against
+        // 130 here). Terms: the launches, the k steps of the rounds of blocks (rounding, S^2 matrix
+        // instructions per tile, dY by single values), the parts' sums, the maxima's reads and their
+        // taps, the patches' copies, the maxima's groups, dY's reads by every position tile.
+        const double steps = std::ceil(tiles * p.parts / slots) * p.per_part * p.KS, s9 = S * S / 9.0, M = 1.0e6;
+        const double xs = (double)p.N * p.C * p.H * p.W, dys = (double)p.N * p.F * p.OH * p.OW;
+        const double us = 12.0 + (0.25 + (p.tf == 2 ? 0.73 : 0.18) * s9 + (p.OW % 4 ? 0.26 : 0.0)) * steps +
+                          5.0 * outs * p.parts / M + 1.2 * (xs + dys) / M +
+                          0.017 * std::ceil(tiles * p.parts / slots) * p.per_part * p.pxgroups * nch +
+                          300.0 * p.C * p.xgroups * p.pgroups * p.T / M + 0.2 * p.T + 0.065 * p.xgroups * p.pgroups +
+                          0.29 * p.ptiles * dys / M;
+        if (us > 0.97 * conv_pipeline_us(RG_CONV_GRAD_WEIGHT, s, S, num_cus)) return false;
+    }
     p.dT = make_fastdiv((uint32_t)p.T);
     p.dTW = make_fastdiv((uint32_t)p.TW);
     p.dOH = make_fastdiv((uint32_t)p.OH);

@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "repro_gemm_math.h"
+#include "rg_conv_cost.h"
 #include "rg_digits.h"
 #include "rg_internal.h"
 #include "rg_mfma.h"
@@ -995,17 +996,6 @@ bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, bool force
         }
     }
     if (p.patch) p.nwf = 1;
-    // Few source channels leave most of a group of 16 idle, and few output channels most of a tile
-    // of 32: the GEMM pipeline (k or output rows (channel, tap), padded to 64) then has the fewer
-    // matrix operations.
-    const double kpad = 16.0 * ceil_div(p.C, 16) * T;
-    if (dx) {
-        const double here = (double)s.N * s.H * s.W * 32 * ceil_div(p.F, 32) * kpad / (s.SY * s.SX);
-        const double gemm = (double)s.N * OH * OW * (64.0 * ceil_div(s.C * T, 64)) * (64.0 * ceil_div(s.F, 64));
-        if (here > 6.0 * gemm && !forced) return false;
-    } else if (!forced && kpad > (p.patch ? 2.25 : 1.5) * 64.0 * ceil_div(s.C * T, 64)) {
-        return false;
-    }
     const int bf = 32 * p.tf * p.nwf;
     p.ftiles = ceil_div(p.F, bf);
     const int Fp = p.ftiles * bf;
@@ -1099,13 +1089,26 @@ bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, bool force
         }
     }
     if ((long long)p.blocks * p.split > INT_MAX / 2) p.split = 1;
-    // The forward pass's GEMM pipeline slices its windows in one launch while they fit the one-pass
-    // slicing and then splits along k at its own best tile, which is faster where this kernel needs
-    // parts (8 x 256 x 14 x 14, 256 filters 3x3: 35 us against 40), and where windows overlap but
-    // not at stride 1, so that every value is fetched and rounded once per tap (32 x 128 x 28 x 28,
-    // 128 filters 3x3, stride 2: 35 against 44). Longer windows it packs first (32 x 512 x 7 x 7,
-    // 512 filters: 81 against 66 here).
-    if (!forced && !dx && (p.split > 1 || (!p.patch && T > 1)) && s.C * T <= ONEPASS_MAX_K) return false;
+    if (!forced) {
+        // Against the GEMM pipeline (rg_conv_cost.h: how both were fitted, and what it replaced). Terms:
+        // the launches, rounds of blocks and their steps (rounding, and S^2 matrix instructions per
+        // tile; less where a compute unit has one block), the weights' slicing per unit of 16 k, the
+        // maxima's read, the outputs' stores, the parts' sums, the length of a sum. (An input
+        // gradient is mostly twice as fast here, and the pipeline's estimate the coarser one.)
+        const bool lone = p.blocks * (double)p.split <= num_cus, wide = p.tf == 2;
+        const double rounds = std::ceil(p.blocks * (double)p.split / slots), steps = rounds * ceil_div(stages, p.split);
+        const double s9 = S * S / 9.0, units = q / (16.0 * S), source = (double)p.N * p.C * p.H * p.W, M = 1.0e6;
+        double us;
+        if (p.patch)
+            us = 8.9 + 0.83 * dx + 2.6 * rounds +
+                 (lone ? 0.38 + (wide ? 1.2 : 0.43) * s9 : 0.57 + (wide ? 1.2 : 0.7) * s9) * steps + 43.0 * units / M +
+                 1.0 * source / M + 1.6 * outs / M + (p.split > 1 ? 2.9 + 4.9 * outs * p.split / M : 0.0) + 0.081 * stages;
+        else
+            us = 10.0 + 1.9 * dx + 1.2 * rounds +
+                 (lone ? 0.75 + (wide ? 1.5 : 0.46) * s9 : 0.8 + (wide ? 1.4 : 1.1) * s9) * steps + 46.0 * units / M +
+                 0.67 * source / M + 1.5 * outs / M + (p.split > 1 ? 3.0 + 4.7 * outs * p.split / M : 0.0) + 0.071 * stages;
+        if (us > (dx ? 1.03 : 1.0) * conv_pipeline_us(kind, s, S, num_cus)) return false;
+    }
     p.dblocks = make_fastdiv((uint32_t)p.blocks);
     p.dOPL = make_fastdiv((uint32_t)p.OPL);
     p.dF = make_fastdiv((uint32_t)p.F);

@@ -99,6 +99,11 @@ int rg_conv2d_algo_ws(int pass, const float* a, const float* b, float* out, cons
  * (invalid value) for a null argument, an unknown pass or an invalid shape. */
 int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int* info);
 
+/* The same for info[0 .. 10], with `forced` the plan of RG_CONV_ALGO_FUSED. info[8]: taps of the first
+ * class (weight gradient: k steps per chunk); info[9]: its stages (chunks per part); info[10]: groups
+ * of 16 source channels (chunks). */
+int rg_test_conv_plan(int pass, const rg_conv_shape* g, int S, int num_cus, int forced, int* info);
+
 #ifdef __cplusplus
 }
 #endif

@@ -14,11 +14,12 @@ BLOCK = 128       # positions per block
 PATCH = 384       # values per channel and slot
 
 
-def fused(pass_, shape, S=3, num_cus=256):
-    info = (ctypes.c_int * 8)()
+def fused(pass_, shape, S=3, num_cus=256, forced=False):
+    info = (ctypes.c_int * 11)()
     g = rg.ConvShape(*shape).to_c()
-    assert _lib.lib.rg_test_conv_fused(pass_, ctypes.byref(g), S, num_cus, info) == 0, shape
-    return dict(zip(("taken", "patch", "split", "classes", "strips", "width", "groups", "tf"), info))
+    assert _lib.lib.rg_test_conv_plan(pass_, ctypes.byref(g), S, num_cus, int(forced), info) == 0, shape
+    return dict(zip(("taken", "patch", "split", "classes", "strips", "width", "groups", "tf", "taps",
+                     "stages", "channel_groups"), info))
 
 
 def test_routes():
@@ -30,12 +31,23 @@ def test_routes():
     assert not fused(DW, (32, 512, 7, 7, 512, 3, 3, 1, 1, 1, 1))["taken"]    # many filters, few windows
     assert not fused(DW, (8, 64, 20, 20, 64, 3, 3, 3, 3, 1, 1))["taken"]     # column stride 3
     strided = (32, 64, 56, 56, 128, 3, 3, 2, 2, 1, 1)
-    assert not fused(FWD, strided)["taken"]             # overlapping windows, not at stride 1
     p = fused(DX, strided)
     assert p["taken"] and not p["patch"] and p["classes"] == 4
     assert fused(FWD, (32, 64, 56, 56, 256, 1, 1, 1, 1, 0, 0))["taken"]
-    assert not fused(FWD, (8, 256, 14, 14, 256, 3, 3, 1, 1, 1, 1))["taken"]   # needs parts
-    assert fused(FWD, (32, 512, 7, 7, 512, 3, 3, 1, 1, 1, 1))["split"] > 1    # past one-pass slicing
+    # Measured on both routes (us, fused against the pipeline):
+    assert fused(FWD, strided)["taken"]                                       # 44, 56
+    assert fused(FWD, (32, 512, 7, 7, 512, 3, 3, 1, 1, 1, 1))["split"] > 1    # 71, 81
+    assert fused(FWD, (100, 6, 14, 14, 16, 5, 5, 1, 1, 0, 0))["taken"]        # 18.1, 18.9
+    for shape in ((8, 256, 14, 14, 256, 3, 3, 1, 1, 1, 1),                    # 43, 37
+                  (32, 128, 28, 28, 128, 3, 3, 2, 2, 1, 1),                   # 47, 36
+                  (1, 64, 56, 56, 256, 3, 3, 1, 1, 1, 1),                     # 28, 24
+                  (22, 828, 8, 8, 51, 7, 7, 2, 2, 0, 0),                      # 119, 42
+                  (3, 750, 8, 7, 1714, 5, 5, 2, 2, 2, 2),                     # 238, 95
+                  (1, 1149, 7, 9, 933, 5, 5, 1, 1, 2, 2)):                    # 220, 88
+        assert not fused(FWD, shape)["taken"] and fused(FWD, shape, forced=True)["taken"], shape
+    for shape in ((3, 1068, 14, 14, 53, 7, 7, 2, 2, 3, 3),                    # 92, 53
+                  (2, 35, 10, 10, 124, 7, 7, 1, 1, 0, 0)):                    # 29, 22
+        assert not fused(DW, shape)["taken"] and fused(DW, shape, forced=True)["taken"], shape
     assert not fused(FWD, (32, 3, 112, 112, 64, 7, 7, 2, 2, 3, 3))["taken"]   # 3 channels
     assert not fused(DX, (8, 8, 20, 20, 16, 5, 5, 3, 3, 2, 2))["taken"]       # nine classes
     bad = rg.ConvShape(1, 1, 3, 3, 1, 5, 5).to_c()      # kernel larger than the image
@@ -52,7 +64,7 @@ def patch_shapes(count):
         h, w = rng.randint(k[0], 90), rng.randint(k[1], 150)
         shape = (n, c, h, w, f, k[0], k[1], 1, 1, rng.randint(0, k[0] - 1), rng.randint(0, k[1] - 1))
         for pass_ in (FWD, DX):
-            p = fused(pass_, shape)
+            p = fused(pass_, shape, forced=True)
             if p["patch"]:
                 count -= 1
                 yield pass_, shape, p
@@ -103,7 +115,7 @@ def test_weight_gradient_chunks_fit_every_block():
         h, w = rng.randint(k[0], 90), rng.randint(k[1], 300)
         sy, sx = rng.choice([1, 1, 2, 3]), rng.choice([1, 1, 2])
         shape = (n, c, h, w, f, k[0], k[1], sy, sx, rng.randint(0, k[0] - 1), rng.randint(0, k[1] - 1))
-        p = fused(DW, shape)
+        p = fused(DW, shape, forced=True)
         if not p["taken"]:
             continue
         found += 1

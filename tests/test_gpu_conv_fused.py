@@ -87,7 +87,7 @@ def test_gathered_taps_match_oracle(torch_gpu, S):
 
 
 def test_shapes_cover_the_routes():
-    plans = [(p, fused(p, s)) for s in SHAPES for p in (FWD, DX)]
+    plans = [(p, fused(p, s, forced=True)) for s in SHAPES for p in (FWD, DX)]
     for pass_ in (FWD, DX):
         mine = [f for p, f in plans if p == pass_ and f["taken"]]
         assert any(f["patch"] and f["split"] == 1 for f in mine)
@@ -95,8 +95,12 @@ def test_shapes_cover_the_routes():
         assert any(not f["patch"] for f in mine)
         assert any(f["strips"] > 1 for f in mine)
         assert {f["tf"] for f in mine} == {1, 2}
-    mine = [(s, f) for s in SHAPES for f in [fused(DW, s)] if f["taken"]]
+    mine = [(s, f) for s in SHAPES for f in [fused(DW, s, forced=True)] if f["taken"]]
     assert len(mine) >= 10 and any(f["strips"] > 1 for _, f in mine) and {f["tf"] for _, f in mine} == {1, 2}
+    gathers = [fused(FWD, s, forced=True) for s in GATHERS]
+    assert all(f["taken"] and not f["patch"] for f in gathers)
+    for several_taps, parts in ((True, False), (True, True), (False, True)):
+        assert any((f["taps"] > 1) == several_taps and (f["split"] > 1) == parts for f in gathers)
     assert {s[8] for s, _ in mine} == {1, 2} and any((s[3] + 2 * s[10] - s[6]) // s[8] % 4 != 3 for s, _ in mine)
 
 

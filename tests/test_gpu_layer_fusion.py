@@ -8,6 +8,7 @@ import torch
 import bit_reproducible_training_amd as rg
 from bit_reproducible_training_amd import _lib
 from bit_reproducible_training_amd._lib import _backend, lib
+from test_conv_fused_plan import FWD, fused
 
 pytestmark = pytest.mark.gpu
 
@@ -65,8 +66,8 @@ def test_bias_entry_point_over_algorithms(algo, split_k):
     assert lib.rg_gemm_bias_fp32_ws(A.data_ptr(), B.data_ptr(), None, *args) == 1
 
 
-# (N, C, H, W, F, K, stride, padding): direct, window gather (1x1 and strided), patch, split
-# reduction, the GEMM pipeline, one output pixel, channel counts off the tiles.
+# (N, C, H, W, F, K, stride, padding): direct, window gather (1x1), patch, the GEMM pipeline, one output
+# pixel, channel counts off the tiles. The route that each of CONV_ROUTES takes is asserted beside it.
 CONVS = [(100, 6, 14, 14, 16, 5, 1, 0), (2, 3, 9, 9, 5, 3, 1, 1), (4, 64, 28, 28, 70, 1, 1, 0),
          (4, 64, 28, 28, 128, 3, 2, 1), (4, 64, 28, 28, 64, 3, 1, 1), (3, 40, 17, 19, 33, 3, 1, 1),
          (2, 512, 7, 7, 512, 3, 1, 1), (8, 256, 14, 14, 256, 3, 2, 0), (64, 16, 5, 5, 120, 5, 1, 0)]
@@ -80,6 +81,24 @@ def test_conv_bias_is_one_addition_after_the_convolution(shape, S):
     x, w, b = torch.randn(N, C, H, W, device="cuda"), torch.randn(F, C, K, K, device="cuda"), _bias(F)
     want = rg.conv2d(x, w, s, s, p, p, S) + b.view(1, -1, 1, 1)
     assert torch.equal(_bits(_backend.conv2d_bias(x, w, b, s, s, p, p, S)), _bits(want))
+
+
+# The same with its route: (holds patches, has parts along k, several taps), the window gather's and the
+# patches' reductions of parts among them; None: the GEMM pipeline.
+CONV_ROUTES = [((16, 64, 28, 28, 8, 2, 2, 1), (0, False, True)), ((8, 64, 28, 28, 33, 1, 1, 0), (0, False, False)),
+               ((1, 4200, 3, 3, 33, 1, 2, 0), (0, True, False)), ((1, 512, 3, 3, 33, 3, 2, 1), (0, True, True)),
+               ((8, 64, 28, 28, 33, 2, 1, 1), (1, False, True)), ((1, 1024, 3, 3, 33, 2, 1, 1), (1, True, True)),
+               ((4, 64, 28, 28, 128, 3, 2, 1), None), ((1, 750, 8, 7, 200, 5, 2, 2), None)]
+
+
+@pytest.mark.parametrize("shape,route", CONV_ROUTES)
+@pytest.mark.parametrize("S", [1, 3])
+def test_conv_bias_on_every_route(shape, route, S):
+    N, C, H, W, F, K, s, p = shape
+    plan = fused(FWD, (N, C, H, W, F, K, K, s, s, p, p))
+    taken = (plan["patch"], plan["split"] > 1, plan["taps"] > 1) if plan["taken"] else None
+    assert taken == route
+    test_conv_bias_is_one_addition_after_the_convolution(shape, S)
 
 
 # (A, B, C) of sums over A and C: columns and segments, one chunk and several, few and many.
