@@ -561,9 +561,10 @@ bool dw_plan(const rg_conv_shape& s, int S, int num_cus, bool forced, DwPlan* ou
     const int nch = std::min(p.C, (DW_POS - 2 + p.T) / p.T + 1);
     // Strips and chunks: the widest strips whose patch fits with the fewest dead quads.
     double best = 0.0;
-    for (int ns = 1; ns <= p.OW; ++ns) {
-        const int sw = ceil_div(ceil_div(p.OW, ns), 4) * 4, sq = sw / 4;
-        if (ns > 1 && (ns - 1) * sw >= p.OW) continue;
+    for (int w = ceil_div(std::min(p.OW, 64 * DW_GROUPS), 4) * 4; w >= 4;) {
+        // (width w from the widest that can fit, with the fewest strips it takes)
+        const int ns = ceil_div(p.OW, w), sw = ceil_div(ceil_div(p.OW, ns), 4) * 4, sq = sw / 4;
+        w = sw - 4;
         const double cols = (double)p.OW / ((double)ns * sw);
         const int pw = (sw - 1) * p.SX + p.TW;
         for (int rc = 1; rc <= 32; ++rc) {
@@ -600,14 +601,20 @@ bool dw_plan(const rg_conv_shape& s, int S, int num_cus, bool forced, DwPlan* ou
     const int max_chunks = std::max(1, (S == 3 ? 44352 : S == 2 ? 66560 : 133120) / (32 * p.KS));
     const double tiles = (double)p.ptiles * p.ftiles, slots = 2.0 * num_cus, outs = (double)p.F * p.K;
     double cost = -1.0;
-    for (int per = 1; per <= std::min(p.chunks, max_chunks); ++per) {
+    // (Only the shortest part of each number of parts, until one round of blocks alone takes longer:
+    // of all lengths 2-6 us of host time a call, of these 0.7-1.3.)
+    for (int per = 1; per <= std::min(p.chunks, max_chunks);) {
         const int parts = ceil_div(p.chunks, per);
-        const double t = std::ceil(tiles * parts / slots) * (8.0 + 1.45 * per * p.KS) + outs * 16.0 * parts / 4.0e6;
+        const double round = 8.0 + 1.45 * per * p.KS;
+        if (cost >= 0.0 && round >= cost) break;
+        const double t = std::ceil(tiles * parts / slots) * round + outs * 16.0 * parts / 4.0e6;
         if (cost < 0.0 || t < cost) {
             cost = t;
             p.per_part = per;
             p.parts = parts;
         }
+        if (parts == 1) break;
+        per = ceil_div(p.chunks, parts - 1);
     }
     if (tiles * p.parts >= 1073741824.0) return false;
     // Maxima: enough blocks to keep the memory busy.

@@ -3,6 +3,7 @@ kernel relies on (a block's patch fits its LDS slot wherever the block starts; a
 slot is free, and the next patch in it ready, before its first use)."""
 import ctypes
 import random
+import time
 
 import pytest
 
@@ -161,3 +162,17 @@ def test_forced_algorithms_are_known():
         except rg.ReproGemmError as e:
             code = e.code
         assert (code != 1) == known, algo  # (without a GPU a known one stops at the device query)
+
+
+@pytest.mark.parametrize("pass_", [FWD, DW, DX])
+@pytest.mark.parametrize("S", [1, 3])
+def test_planning_wide_rows_takes_microseconds(pass_, S):
+    """A call plans twice, so the search for strips and parts has to stay far below a launch (a search
+    by every number of strips took 2 ms here, by every length of a part 5 us)."""
+    for shape in ((1, 2, 31, 1000000, 4, 31, 31, 1, 1, 0, 0), (64, 64, 1, 16384, 64, 1, 3, 1, 1, 0, 1)):
+        best = 1.0
+        for _ in range(20):
+            t = time.perf_counter()
+            fused(pass_, shape, S)
+            best = min(best, time.perf_counter() - t)
+        assert best < 2e-4, (shape, best)
