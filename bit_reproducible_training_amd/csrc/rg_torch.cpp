@@ -64,13 +64,13 @@ Tensor workspace_like(size_t bytes, const Tensor& t) {
 }
 
 // A layer's bias (or none) that a library call can add in its own launches: n contiguous floats on
-// the operands' device. Any other (a broadcastable shape, another type or stride) is added by a
-// PyTorch operation.
+// the operands' device. Any other (a broadcastable shape, another type or stride, a lazily negated
+// view, whose memory holds the opposite values) is added by a PyTorch operation.
 const float* fusible_bias(const c10::optional<Tensor>& bias, const Tensor& a, int64_t n) {
     if (!bias.has_value()) return nullptr;
     const Tensor& b = *bias;
     const bool ok = b.scalar_type() == torch::kFloat32 && b.device() == a.device() && b.dim() == 1 &&
-                    b.size(0) == n && b.is_contiguous();
+                    b.size(0) == n && b.is_contiguous() && !b.is_neg();
     return ok ? b.data_ptr<float>() : nullptr;
 }
 

@@ -48,6 +48,18 @@ def test_linear_bias_is_one_addition_after_the_gemm(M, N, K, S):
     assert torch.equal(_bits(_backend.linear(x, w, one, M, N, K, S)), _bits(want))
 
 
+def test_a_lazily_negated_bias_is_its_value():
+    """A negated view's memory holds the opposite values; the layers' biases may be such views."""
+    x, w, b = torch.randn(5, 40, device="cuda"), torch.randn(8, 40, device="cuda"), _bias(8)
+    neg = torch._neg_view(b)
+    assert neg.is_neg() and neg.is_contiguous()
+    want = rg.gemm(x, w, 5, 8, 40, False, True, 3) + neg
+    assert torch.equal(_bits(_backend.linear(x, w, neg, 5, 8, 40, 3)), _bits(want))
+    xc, wc = torch.randn(2, 3, 6, 6, device="cuda"), torch.randn(8, 3, 3, 3, device="cuda")
+    want = rg.conv2d(xc, wc, 1, 1, 0, 0, 3) + neg.view(1, -1, 1, 1)
+    assert torch.equal(_bits(_backend.conv2d_bias(xc, wc, neg, 1, 1, 0, 0, 3)), _bits(want))
+
+
 @pytest.mark.parametrize("algo", list(rg.Algo))
 @pytest.mark.parametrize("split_k", [1, 3])
 def test_bias_entry_point_over_algorithms(algo, split_k):
