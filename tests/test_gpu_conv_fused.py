@@ -86,6 +86,35 @@ def test_gathered_taps_match_oracle(torch_gpu, S):
         assert np.array_equal(got, _oracle("fwd", x, w, shape, S).view(np.uint32).ravel()), (shape, S)
 
 
+# Planes and rows of whole quads, which the weight gradient reads by 16-byte loads from aligned bases.
+QUADS = [(2, 16, 8, 8, 16, 3, 3, 1, 1, 1, 1), (3, 9, 12, 16, 40, 3, 3, 1, 1, 1, 1),
+         (2, 17, 17, 32, 33, 3, 4, 2, 2, 1, 1), (1, 20, 4, 64, 6, 1, 1, 1, 1, 0, 0)]
+
+
+@pytest.mark.parametrize("offset_a,offset_b", [(0, 0), (1, 0), (0, 1), (1, 3)])
+def test_bases_off_16_bytes(torch_gpu, offset_a, offset_b):
+    """Operands that start 0, 4 or 12 bytes past a 16-byte boundary: the loads by quads of either
+    operand, or of both, give way to single ones."""
+    torch = torch_gpu
+    stream = torch.cuda.current_stream().cuda_stream
+    assert any(fused(DW, s, forced=True)["taken"] and O.conv_out_hw(s)[1] % 4 == 0 for s in QUADS)
+    for shape in QUADS:
+        g = RC.ConvShape(*shape)
+        x, w, dy = _inputs(shape, 31)
+        for kind, p, a, b in (("fwd", RC.FORWARD, x, w), ("dW", RC.GRAD_WEIGHT, dy, x), ("dX", RC.GRAD_INPUT, dy, w)):
+            want = _oracle(kind, a, b, shape, 3).view(np.uint32).ravel()
+            da, db = (torch.empty(v.size + 4, device="cuda")[o:o + v.size].copy_(torch.from_numpy(v))
+                      for v, o in ((a, offset_a), (b, offset_b)))
+            assert da.data_ptr() % 16 == 4 * offset_a and db.data_ptr() % 16 == 4 * offset_b
+            for algo in (RC.ALGO_FUSED, RC.ALGO_PIPELINE):
+                note("conv bases", kind, shape, offset_a, offset_b, "algo=%d" % algo)
+                out = torch.full((want.size,), float("nan"), device="cuda")
+                ws = torch.empty(RC.conv2d_algo_workspace(p, g, 3, algo), dtype=torch.uint8, device="cuda")
+                assert RC.repro_conv2d_algo_ws(p, da.data_ptr(), db.data_ptr(), out.data_ptr(), g, 3, algo,
+                                               ws.data_ptr(), ws.numel(), stream) == 0
+                assert np.array_equal(out.cpu().numpy().view(np.uint32), want), (kind, shape, algo)
+
+
 def test_shapes_cover_the_routes():
     plans = [(p, fused(p, s, forced=True)) for s in SHAPES for p in (FWD, DX)]
     for pass_ in (FWD, DX):

@@ -165,3 +165,51 @@ def test_conv_replays_equal_eager(torch_gpu):
     torch.cuda.synchronize()
     for o, exp in zip((y, dw, dx), want()):
         assert np.array_equal(_bits(o).reshape(-1), exp.reshape(-1))
+
+
+# Shapes (N, C, H, W, F, KH, KW, SY, SX, PY, PX): patches, patches with parts along k, gathers with
+# and without parts, residue classes of the input gradient, several parts of the weight gradient.
+FUSED_SHAPES = [(2, 16, 14, 14, 33, 3, 3, 1, 1, 1, 1), (1, 512, 7, 7, 40, 3, 3, 1, 1, 1, 1),
+                (1, 512, 7, 7, 40, 3, 3, 2, 2, 1, 1), (2, 32, 20, 20, 70, 1, 1, 1, 1, 0, 0)]
+
+
+@pytest.mark.parametrize("shape", FUSED_SHAPES)
+def test_fused_convolution_replays_equal_eager(torch_gpu, shape):
+    """The implicit GEMMs of the three passes in one graph, on inputs and a workspace that eager work
+    changes between the replays."""
+    torch = torch_gpu
+    RC = rg.repro_conv
+    g_ = RC.ConvShape(*shape)
+    torch.manual_seed(5)
+    x = torch.randn(g_.N, g_.C, g_.H, g_.W, device="cuda")
+    w = 0.1 * torch.randn(g_.F, g_.C, g_.KH, g_.KW, device="cuda")
+    dy = 1e-3 * torch.randn(g_.N, g_.F, g_.OH, g_.OW, device="cuda")
+    y, dw, dx = torch.empty_like(dy), torch.empty_like(w), torch.empty_like(x)
+    passes = [(RC.FORWARD, x, w, y), (RC.GRAD_WEIGHT, dy, x, dw), (RC.GRAD_INPUT, dy, w, dx)]
+    wss = [torch.empty(RC.conv2d_algo_workspace(p, g_, 3, RC.ALGO_FUSED), dtype=torch.uint8, device="cuda")
+           for p, _, _, _ in passes]
+
+    def call():
+        for (p, a, b, o), ws in zip(passes, wss):
+            assert RC.repro_conv2d_algo_ws(p, a.data_ptr(), b.data_ptr(), o.data_ptr(), g_, 3, RC.ALGO_FUSED,
+                                           ws.data_ptr(), ws.numel(),
+                                           torch.cuda.current_stream().cuda_stream) == 0
+
+    note("graph fused conv", shape)
+    g = _capture(torch, call)
+    for rep in range(3):
+        if rep:
+            x.copy_(torch.randn_like(x) * 7.0 ** rep)
+            dy.copy_(torch.randn_like(dy))
+            w.mul_(-1.5)
+        for o in (y, dw, dx):
+            o.fill_(float("nan"))
+        for ws in wss:
+            ws.fill_(255 if rep == 1 else 0)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        xn, wn, dyn = (t.cpu().numpy().reshape(-1) for t in (x, w, dy))
+        for o, want in ((y, O.conv2d(xn, wn, shape, 3)), (dw, O.conv2d_grad_weight(dyn, xn, shape, 3)),
+                        (dx, O.conv2d_grad_input(dyn, wn, shape, 3))):
+            assert np.array_equal(_bits(o).reshape(-1), want.view(np.uint32).reshape(-1)), rep
