@@ -164,6 +164,8 @@ _SIGNATURES = {
                                           ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
     "rg_test_conv_plan": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape), ctypes.c_int,
                                          ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
+    "rg_test_conv_schedule": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                             ctypes.c_int, ctypes.POINTER(ctypes.c_int)]),
     "rg_conv2d_algo": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape), ctypes.c_int,
                                       ctypes.POINTER(ctypes.c_int)]),
     "rg_conv2d_algo_workspace": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(rg_conv_shape),

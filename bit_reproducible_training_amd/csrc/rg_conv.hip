@@ -1067,6 +1067,18 @@ int rg_test_conv_plan(int pass, const rg_conv_shape* g, int S, int num_cus, int 
     return hipSuccess;
 }
 
+int rg_test_conv_schedule(int pass, int T, int s0, int s1, int groups, int* copied) {
+    if (!copied || !rg::valid_pass(pass) || T < 1 || s0 < 0 || s1 <= s0 || groups < 1) return hipErrorInvalidValue;
+    for (int g = 0; g < groups; ++g) copied[g] = -2;
+    const bool dw = pass == RG_CONV_GRAD_WEIGHT;
+    int next = dw ? 0 : 4 * s0 / T, end = dw ? groups : std::min(groups, (4 * s1 - 1) / T + 1);
+    const int first = dw ? 2 : rg::patch_first(s0);
+    for (int i = 0; i < first && next < end; ++i) copied[next++] = -1;
+    for (int s = s0; s < s1; ++s)
+        if (next < end && (dw ? rg::dw_due(next, T, s) : rg::patch_due(next, T, s))) copied[next++] = s;
+    return hipSuccess;
+}
+
 int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int* info) {
     if (!info) return hipErrorInvalidValue;
     int all[11];

@@ -29,6 +29,11 @@ struct DwPlan {
     size_t xmax, dmax, ea, eb, part, total;  // workspace offsets
 };
 
+// Schedule of dw_contract's two patch slots: whether chunk c >= 2 is copied (and table c + 2 built)
+// during stage s, all KS steps of chunk c - 2 lying before it. That comes a stage before chunk c's own
+// first, floor(c KS / 2), for KS >= 2.
+__host__ __device__ inline bool dw_due(int c, int KS, int s) { return (c - 1) * KS <= 2 * s; }
+
 // Fills *plan and returns true when the fused kernels take this weight gradient (a valid shape): where
 // they are faster than the GEMM pipeline, or with `forced` wherever they can.
 bool dw_plan(const rg_conv_shape& s, int S, int num_cus, bool forced, DwPlan* plan);

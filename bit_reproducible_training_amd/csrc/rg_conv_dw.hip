@@ -193,8 +193,7 @@ dw_maxima(DwPlan p, const float* __restrict__ x, const float* __restrict__ dy, c
 
 // The contraction. Wavefront w: positions 32 w .. 32 w + 31 of the block's 128 x 32 TF filters, two k
 // steps of 32 per stage. Chunk c of the part (its RC output rows' source rows) sits in patch slot
-// c % 2; chunk c + 2 is copied during the first stage that starts past chunk c's last step,
-// ceil((c + 1) KS / 2), before its own first, floor((c + 2) KS / 2), for KS >= 2. The quads' offsets
+// c % 2, the first two copied before the first stage and the others as dw_due says. The quads' offsets
 // (into dY and into the patch) are a table per chunk, in ring slot c % 4: table c + 2 is built when
 // chunk c is copied (chunk c - 2, whose slot it takes, is done), at least a stage before dY's loads,
 // which go out two stages ahead, look into it.
@@ -470,7 +469,7 @@ dw_contract(DwPlan p, const float* __restrict__ dy, const float* __restrict__ x,
         publish(stages > 1);
         int next = 2;
         for (int s = 0; s < stages; ++s) {
-            if (next < nchunks && (next - 1) * p.KS <= 2 * s) {
+            if (next < nchunks && dw_due(next, p.KS, s)) {
                 copy_patch(next);
                 build_table(next + 2);
                 ++next;

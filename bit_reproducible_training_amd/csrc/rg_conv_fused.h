@@ -60,6 +60,14 @@ struct FusedPlan {
     size_t q, ef, maxima, imax, ew, part, total;  // workspace offsets
 };
 
+// Schedule of fused_patch's two patch slots (channel group cg in slot cg % 2), for a part of k from
+// stage s0 on: how many groups, from the first it reads on, are copied before its first stage, and
+// whether a later group cg is copied during stage s (at most one a stage): its slot is free, the last k
+// group of cg - 2 lying before the stage. That comes a stage before cg's own first, floor(cg T / 4),
+// for T = 4 and for every T >= 6 taps.
+__host__ __device__ inline int patch_first(int s0) { return s0 > 0 ? 2 : 1; }
+__host__ __device__ inline bool patch_due(int cg, int T, int s) { return cg < 2 || (cg - 1) * T <= 4 * s; }
+
 // Fills *plan and returns true when the fused kernels take this pass (kind: RG_CONV_FORWARD or
 // RG_CONV_GRAD_INPUT; the shape is valid): where they are faster than the GEMM pipeline, or with
 // `forced` wherever they can.

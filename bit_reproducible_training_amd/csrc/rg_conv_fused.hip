@@ -631,9 +631,7 @@ fused_contract(FusedPlan p, const float* __restrict__ src, const char* __restric
 // MFMA's operand registers (lane l: position l % 32, the 16 channels of k group 2 i + l / 32), so
 // the digits never go through LDS. Positions run over (image, column strip, row, column): strips
 // narrow wide images until a block's patch fits PX values per channel.
-// Patch slots: channel group cg in slot cg % 2; group cg + 2 is copied in during the first stage
-// after the last that reads cg, stage ceil((cg + 1) T / 4), which comes before its own first stage,
-// floor((cg + 2) T / 4), for T = 4 and for every T >= 6.
+// Patch slots: channel group cg in slot cg % 2, copied as patch_first and patch_due say.
 // LDS: 2 x 16 x 384 x 4 B of patches and two stages of 64 output channels' panels, 74 KB: two
 // blocks of 4 wavefronts share a compute unit.
 template <int S, int TF, bool FORWARD>
@@ -758,7 +756,7 @@ fused_patch(FusedPlan p, const float* __restrict__ src, const char* __restrict__
             patch_offsets();
             copy_patch(cg0);
             // (a part that starts in cg0's last groups reads the next group's patch at once)
-            if (s0 > 0 && cg0 + 1 < cgroups) copy_patch(cg0 + 1);
+            if (patch_first(s0) > 1 && cg0 + 1 < cgroups) copy_patch(cg0 + 1);
             __builtin_amdgcn_sched_barrier(0);
         };
         if (FORWARD) {
@@ -867,14 +865,14 @@ fused_patch(FusedPlan p, const float* __restrict__ src, const char* __restrict__
     // which run on their own (the fences keep that order).
     auto pipeline = [&](auto FAST) RG_INLINE {
         constexpr int EVERY = S == 3 ? 2 : 1;
-        int next_cg = s0 > 0 ? cg0 + 2 : 1;
+        int next_cg = cg0 + patch_first(s0);
         for (int s = s0; s < s1; ++s) {
             float v[16], v1[16];
             v4i d0[S], d1[S], fa[S][TF];
             read_values(v, s, 0);
             read_panels(fa, s, 0);
             if (s + 1 < s1) copy_panels(s + 1);
-            if (next_cg < cgroups && (next_cg < 2 || (next_cg - 1) * c.T <= 4 * s)) {
+            if (next_cg < cgroups && patch_due(next_cg, c.T, s)) {
                 copy_patch(next_cg);
                 ++next_cg;
             }

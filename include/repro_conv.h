@@ -104,6 +104,12 @@ int rg_test_conv_fused(int pass, const rg_conv_shape* g, int S, int num_cus, int
  * of 16 source channels (chunks). */
 int rg_test_conv_plan(int pass, const rg_conv_shape* g, int S, int num_cus, int forced, int* info);
 
+/* Test hook (no GPU needed): when the implicit GEMMs copy their source patches. Forward pass and input
+ * gradient with T taps, stages s0 .. s1 - 1 of a part of k: copied[c] is the stage during which channel
+ * group c < groups goes into its slot (-1: before the first, -2: never). Weight gradient with T = k
+ * steps per chunk: the same for its chunks. */
+int rg_test_conv_schedule(int pass, int T, int s0, int s1, int groups, int* copied);
+
 #ifdef __cplusplus
 }
 #endif

@@ -92,17 +92,49 @@ def test_patch_fits_every_block():
             assert values <= p["groups"] * 64, (shape, p, r0)
 
 
+def schedule(pass_, T, s0, s1, groups):
+    copied = (ctypes.c_int * groups)()
+    assert _lib.lib.rg_test_conv_schedule(pass_, T, s0, s1, groups, copied) == 0
+    return list(copied)
+
+
+def test_patches_need_four_or_six_taps():
+    """The slots' schedule serves four taps and six or more; plans hold no patches at others."""
+    seen = set()
+    for kh in range(1, 10):
+        for kw in range(1, 10):
+            for pass_ in (FWD, DX):
+                p = fused(pass_, (4, 64, 20, 20, 64, kh, kw, 1, 1, 0, 0), forced=True)
+                assert p["taken"] and bool(p["patch"]) <= (kh * kw == 4 or kh * kw >= 6), (kh, kw)
+                if p["patch"]:
+                    seen.add(p["taps"])
+    assert 4 in seen and 6 in seen and 5 not in seen and max(seen) > 40
+    for pass_, shape, p in patch_shapes(60):
+        assert p["taps"] == 4 or p["taps"] >= 6, (pass_, shape)
+
+
 @pytest.mark.parametrize("taps", [4] + list(range(6, 82)))
 def test_patch_slots_are_free_and_ready(taps):
     """Stage s reads k groups 4 s .. 4 s + 3, group g channel group g // taps from slot
-    (g // taps) % 2. The kernel copies channel group cg >= 2 during the first stage that starts
-    past the last group of cg - 2; that stage has to come before the first that reads cg."""
-    for cg in range(2, 40):
-        copied = -(-(cg - 1) * taps // 4)
-        assert 4 * copied >= (cg - 1) * taps         # every read of cg - 2 is in an earlier stage
-        assert copied < cg * taps // 4, (taps, cg)
-        if cg > 2:                                   # one copy per stage at most
-            assert copied > -(-(cg - 2) * taps // 4)
+    (g // taps) % 2. Whatever stages a part has, a channel group is copied before the stage that first
+    reads it, and after the last that reads the group before it in its slot."""
+    for groups in (1, 2, 3, 9, 20):
+        stages = -(-groups * taps // 4)
+        starts = sorted({0, 1, 2, 3, taps // 4, stages // 3, stages // 2, stages - 2, stages - 1} - {-1, -2})
+        for s0 in [s for s in starts if 0 <= s < stages]:
+            for s1 in sorted({min(stages, s0 + n) for n in (1, 2, 3, 7, taps, 2 * taps, stages)}):
+                copied = schedule(FWD, taps, s0, s1, groups)
+                reads = {}  # channel group -> first and last stage (a group past the last reads any value)
+                for s in range(s0, s1):
+                    for g in range(4 * s, 4 * s + 4):
+                        if g // taps < groups:
+                            first, _ = reads.get(g // taps, (s, s))
+                            reads[g // taps] = (first, s)
+                for cg, (first, last) in reads.items():
+                    at = copied[cg]
+                    assert at == -1 or s0 <= at < first, (taps, groups, s0, s1, cg)
+                    if cg - 2 in reads:
+                        assert at != -1 and at > reads[cg - 2][1], (taps, groups, s0, s1, cg)
 
 
 def test_weight_gradient_chunks_fit_every_block():
@@ -142,15 +174,33 @@ def test_weight_gradient_chunks_fit_every_block():
 @pytest.mark.parametrize("steps", range(2, 17))
 def test_weight_gradient_slots_are_free_and_ready(steps):
     """Stage s takes k steps 2 s and 2 s + 1, step j chunk j // steps from patch slot (chunk % 2) and
-    table slot (chunk % 4). Chunk c >= 2 is copied, and table c + 2 built, during the first stage
-    that starts past chunk c - 2's last step; chunk c's quads are looked up when dY is loaded, two
-    stages before their own."""
-    for c in range(2, 40):
-        copied = -(-(c - 1) * steps // 2)
-        assert 2 * copied >= (c - 1) * steps and copied < c * steps // 2, (steps, c)
-        if c >= 4:  # tables 0 .. 3 are built before the first stage
-            built = -(-(c - 3) * steps // 2)
-            assert built + 1 <= c * steps // 2 - 2, (steps, c)
+    table slot (chunk % 4). Tables 0 .. 3 are built before the first stage and table c + 2 where chunk c
+    is copied; a chunk's quads are looked up when dY is loaded, two stages before their own."""
+    for chunks in (1, 2, 3, 4, 5, 40):
+        stages = -(-chunks * steps // 2)
+        copied = schedule(DW, steps, 0, stages, chunks)
+        for c in range(chunks):
+            first, last = c * steps // 2, ((c + 1) * steps - 1) // 2
+            if c < 2:
+                assert copied[c] == -1
+            else:
+                assert 0 <= copied[c] < first, (steps, c)
+                assert copied[c] > (((c - 1) * steps) - 1) // 2, (steps, c)   # chunk c - 2 is done
+            if c >= 4:                                                          # table c
+                assert copied[c - 2] >= 0 and copied[c - 2] + 1 <= first - 2, (steps, c)
+
+
+def test_weight_gradient_chunks_take_two_steps_or_more():
+    rng = random.Random(3)
+    seen = set()
+    for _ in range(3000):
+        k = rng.randint(1, 7)
+        shape = (rng.randint(1, 9), rng.randint(1, 64), rng.randint(k, 40), rng.randint(k, 60), rng.randint(1, 64),
+                 k, k, rng.randint(1, 3), rng.randint(1, 2), 0, 0)
+        p = fused(DW, shape, forced=True)
+        if p["taken"]:
+            seen.add(p["taps"])  # (k steps per chunk)
+    assert min(seen) == 2 and max(seen) <= 16 and len(seen) > 5
 
 
 def test_forced_algorithms_are_known():
