@@ -1130,6 +1130,10 @@ bool fused_plan(int kind, const rg_conv_shape& s, int S, int num_cus, bool force
         p.maxima_blocks = ceil_div(pixels, 64);
         maxima = (size_t)pixels * sizeof(uint32_t);
     }
+    // A launch takes fewer than 2^32 work items, the pixels' maxima four a pixel. (The pipeline has no
+    // pass over the pixels: from 2^30 of them on it still takes the strided passes, whose windows are few.)
+    const double first = (double)p.maxima_blocks + (dx ? 0 : p.qblocks), contract = (double)p.blocks * p.split * p.nwf;
+    if (std::max(first, contract) * THREADS >= 4294967296.0) return false;
     p.q = 0;
     p.ef = align_up(p.qbytes);
     p.maxima = p.ef + align_up((size_t)Fp * sizeof(int));

@@ -57,6 +57,16 @@ def test_routes():
     assert _lib.lib.rg_test_conv_fused(7, ctypes.byref(bad), 3, 256, info) == 1
 
 
+def test_plans_keep_to_the_launch_limit():
+    """A launch takes fewer than 2^32 work items; a pass over the pixels takes four for each."""
+    for S in (1, 2):
+        for forced in (False, True):
+            assert not fused(FWD, (2 ** 22, 1, 16, 17, 1, 2, 2, 2, 2, 0, 0), S, forced=forced)["taken"]
+    assert fused(FWD, (2 ** 22, 1, 16, 15, 1, 2, 2, 2, 2, 0, 0), 1, forced=True)["taken"]
+    assert not fused(DX, (2 ** 24, 4, 2, 2, 4, 2, 2, 2, 2, 0, 0), 1, forced=True)["taken"]  # a block per image
+    assert fused(DX, (2 ** 24 - 9, 4, 2, 2, 4, 2, 2, 2, 2, 0, 0), 1, forced=True)["taken"]
+
+
 def patch_shapes(count):
     rng = random.Random(11)
     while count:
