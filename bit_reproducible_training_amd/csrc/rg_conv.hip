@@ -635,7 +635,8 @@ PlanExtras conv_extras(bool raw) {
 // thread's chain of multiply-adds stays short: the direct kernels' time grows with it (MI355X,
 // LeNet-5 at batch 100: forward 11 us at 200 per thread against 33 us for the GEMM pipeline,
 // 28 us at 1200 against 23 us; input gradient 15 us at 150 and 26 us at 400 against 53 and
-// 41 us).
+// 41 us). The limits stand where these two crossed; against the implicit GEMMs the input gradient's
+// is too wide (32 us at 150, but 20 at 400).
 constexpr double DIRECT_AUTO_MACS = 268435456.0;  // 2^28
 constexpr double DIRECT_AUTO_READS = 67108864.0;  // 2^26
 constexpr long long FWD_AUTO_CHAIN = 512;         // K * (padded F) / G multiply-adds per thread
