@@ -244,6 +244,24 @@ def test_gpu_schedule_replay_matches_oracle(hs, flush):
                 assert int(bits(np.float32(got))) == w, (name, lanes, groups, divisor)
 
 
+@pytest.mark.parametrize("divisor", [2, 3, 5, 641, 65535, 65536, 65537, 2 ** 30 - 1, 2 ** 30, 2 ** 30 + 1,
+                                     0x55555555, 2 ** 31 - 2, 2 ** 31 - 1])
+def test_division_by_any_count(hs, divisor):
+    """The division by a shifted reciprocal, digit by digit: quotients of all lengths, remainders of 0, 1
+    and divisor - 1, quotient digits of 0 and 2^32 - 1."""
+    rng = np.random.default_rng(divisor)
+    cases = [x for x in families(rng, 40).values()]
+    for m in (1, divisor - 1, divisor, divisor + 1, divisor * 3, divisor * (2 ** 32 - 1) - 1, divisor << 33):
+        for e in (-149, -101, -37, 0, 31, 64):      # m 2^e as floats of 24 bits each
+            parts = [(m >> k & 0xFFFFFF) * 2.0 ** (k + e) for k in range(0, 72, 24)]
+            cases.append(np.array([sign * p for sign in (1, -1) for p in parts][rng.integers(0, 2) * 3:][:3], np.float32))
+    for x in cases:
+        x = np.ascontiguousarray(x, np.float32)
+        order = np.arange(x.size, dtype=np.int32)
+        got = hs.hs_wide_schedule(x.ctypes.data, order.ctypes.data, x.size, 1, 252, 1, divisor)
+        assert int(bits(np.float32(got))) == exact_bits(x, divisor), (list(x), divisor)
+
+
 def test_gpu_schedule_worst_case_magnitudes(hs):
     """252 adds of the largest wide term into one limb, in both signs, then merges."""
     big = np.full(252 * 64, np.finfo(np.float32).max, np.float32)
