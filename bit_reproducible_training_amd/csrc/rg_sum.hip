@@ -45,6 +45,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 namespace rg {
 namespace {
@@ -160,8 +161,9 @@ struct ThreadSum {
             used = true;
         }
     }
+    // Adds v; the values from `live` on (the same for the whole wave) are zeros.
     template <int N>
-    __device__ __forceinline__ void add(const float (&v)[N]) {
+    __device__ __forceinline__ void add(const float (&v)[N], int live = N) {
         // A NaN is in neither bound; it makes the binary64 sum a NaN, which spill() and the final
         // steps see.
         float m = 0.0f;
@@ -182,7 +184,11 @@ struct ThreadSum {
                 use();
                 uint32_t top_e = 0;
 #pragma unroll
-                for (int i = 0; i < N; ++i) limbs.add(v[i], top_e);
+                for (int g = 0; g < N; g += 4) {
+                    if (g >= live) break;
+#pragma unroll
+                    for (int i = g; i < N && i < g + 4; ++i) limbs.add(v[i], top_e);
+                }
                 nonfinite |= top_e == 0xFFu;
                 since += N;
             }
@@ -204,7 +210,8 @@ struct ThreadSum {
     }
     // Everything into normalised limbs.
     __device__ void finish() {
-        spill();
+        if (count > 0) spill();
+        else use();
         limbs.carry();
     }
 };
@@ -239,15 +246,20 @@ sum_columns(const float* __restrict__ x, int A, int B, int rows_per_chunk, int c
     const int a1 = min(A, a0 + rows_per_chunk);
     ThreadSum sum{LdsAcc{acc + t}};
     if (b < B) {
-        for (int a = a0 + phase; a < a1; a += 4 * BATCH) {
-            float v[BATCH];
+        // A few rows, as every bias gradient of a small batch has, go in a batch of four: in one of 16,
+        // mostly zeros, 11 x 1000000 values took 43 us, of a wide range 66, against 38 and 46.
+        auto rows = [&](int a, auto N) {
+            float v[decltype(N)::value];
 #pragma unroll
-            for (int g = 0; g < BATCH; ++g) {
+            for (int g = 0; g < decltype(N)::value; ++g) {
                 const int r = a + 4 * g;
                 v[g] = r < a1 ? x[(size_t)r * B + b] : 0.0f;
             }
-            sum.add<BATCH>(v);
-        }
+            sum.add<decltype(N)::value>(v, (a1 - a + 3) / 4);
+        };
+        int a = a0 + phase;
+        for (; a + 16 < a1; a += 4 * BATCH) rows(a, std::integral_constant<int, BATCH>());
+        if (a < a1) rows(a, std::integral_constant<int, 4>());
     }
     sum.finish();
     if (watch.flag != nullptr) report(sum.nonfinite != 0, watch.flag, watch.op_id);
